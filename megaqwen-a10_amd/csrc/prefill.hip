@@ -20,23 +20,24 @@
 //   QKV         q|k|v rows on the matrix cores; the epilogue runs QK-norm and RoPE
 //               and writes this layer's K/V cache rows and the rotated queries
 //               (a 128-row tile is one head, so the norm and the rotation pairs
-//               are inside one wave)                        tiles of 32 positions x 128 rows
+//               are inside one wave)                        row tiles of 128 (pf_product)
 //   attention   causal, fp64 on the matrix cores, per (KV head, 8 positions) its 16
 //               queries over cache rows [0, pos0 + p]; a workgroup takes one such
 //               item or two of complementary length, its key blocks cut evenly over
 //               the four waves
 //   digits      of the attention output
-//   O           + residual (the layer input)                 32 positions x 64 rows
+//   O           + residual (the layer input)                 row tiles of 64
 //   digits      post-attention RMSNorm
-//   gate|up     64 channels' gate and up rows per tile; SwiGLU in the epilogue
+//   gate|up     48 channels' gate and up rows per tile; SwiGLU in the epilogue
 //   digits      of the SwiGLU output
-//   down        + residual, bf16: the next layer's input
+//   down        + residual, bf16: the next layer's input     row tiles of 32
 // The last layer stops after its cache rows. The first generated token comes from
 // the decode step of the last prompt token, as in the reference's loop. A phase's work
 // items (positions or product tiles) are dealt round-robin over the workgroups.
 #include <algorithm>
 
 #include "attention.h"
+#include "decode_common.h"
 #include "digits.h"
 
 namespace mq {
@@ -45,8 +46,9 @@ namespace {
 
 constexpr int kFH = 1024, kFI = 3072, kFD = 128, kFQ = 2048, kFNKV = 8;
 constexpr int kFKB = kFI / 64;             // most 64-element K blocks of a product (down: 3072)
-constexpr int kTileP = 32;                 // positions per product tile: 4 waves x 4 pairs
+constexpr int kTileP = 32;                 // positions per product tile: 4 waves x 4 pairs (or 16: x 2 pairs)
 constexpr int kFThreads = 256;
+constexpr int kWtBytes = 128 * 1024;       // most weight bytes a product's row tile holds in LDS
 
 // Chunk workspace for Pp positions (a multiple of kTileP). Digit planes are laid out
 // [K block][position][plane][64 bytes], so that the MFMA A operand of a position pair
@@ -103,8 +105,10 @@ static_assert(sizeof(PfSync) <= 1024, "barrier state");
 
 // LDS of a workgroup, shared by the phases
 struct PfShared {
-    double am[3][kWave][34];               // attention: parts handed to an item's leader wave (m, denominator, outputs)
-    uint4 gb[2][8][kWave];                 // products: a K block's weight operands (B), shared by the waves
+    union {
+        double am[3][kWave][34];           // attention: parts handed to an item's leader wave (m, denominator, outputs)
+        uint4 wt[kWtBytes / 16];           // products: the workgroup's weight rows, as pf_load_weights lays them out
+    };
     double reds[4];
     uint32_t rede[4];
 };
@@ -226,130 +230,157 @@ __device__ void pf_digits(const PfArgs& a, int p, PfShared& sh) {
 }
 
 // ---- products on the int8 matrix cores -------------------------------------------------
-// Work item (row tile rt, position tile pt) of a workgroup of kFThreads threads: wave w takes positions
-// [32 pt + 8 w, +8) (four pairs) and the tile's NT row blocks of 16. Per 64-element K block
-// a wave loads its four A operands (a pair's 8 + 8 digit planes: 1 KB contiguous) and NT B
-// operands (16 weight rows x 64 bytes) and issues 4 NT MFMAs, with the next block's operands
-// in flight. The output tile of pair j, block t: lane l (bit 4 clear) ends with the value of
-// position 2j + l / 32 and weight row 16 t + l % 16 (tile_value).
+// A workgroup keeps one row tile of the product's weights (ROWS rows, whole K) in LDS and runs
+// it against position tiles of 8 NP positions (32 or 16): wave w takes positions [8 NP pt +
+// 2 NP w, +2 NP) (NP pairs). Per 64-element K block a wave reads NT B operands (16 weight rows x
+// 64 bytes) from LDS and issues NP NT MFMAs on its NP A operands (a pair's 8 + 8 digit planes:
+// 1 KB contiguous), which are loaded pf_ring(NP) blocks ahead. The output tile of pair j, block t:
+// lane l (bit 4 clear) ends with the value of position 2j + l / 32 and weight row 16 t + l % 16
+// (tile_value).
 //
-// Row tiles: QKV 32 x 128 rows (q heads 0-15, k heads 0-7, v heads 0-7); O and down
-// 16 x 64 rows; gate|up 48 tiles of 64 channels, blocks 0-3 gate rows, 4-7 up rows.
+// The weights do not depend on the phases before the product, so their loads are issued while
+// the workgroup waits in an earlier grid barrier (pf_load_weights) and cost the product nothing.
+// Loaded inside the K loop, three blocks ahead, every load of a wave waited behind them (loads
+// return in order; ~4 us from HBM): a tile of 16 K blocks took 20-23 us at any prompt length,
+// with 3.4 us of MFMA work. Phases, us at 77 / 512 positions, so loaded -> prefetched into LDS:
+// QKV 22.8 / 41.2 -> 8.6 / 23.6, O 24.5 / 25.3 -> 7.6 / 12.7, gate|up 20.4 / 54.6 -> 9.6 / 30.7, down
+// 30.7 / 31.4 -> 8.6 / 25.9; the whole prefill 4.40 / 6.77 -> 2.80 / 5.36 ms.
+//
+// Row tiles, sized for 128 KB of LDS and for every workgroup to hold one: QKV 32 x 128 rows (a
+// head each: q heads 0-15, k heads 0-7, v heads 0-7); O 16 x 64 rows; gate|up 64 x (48 gate + 48
+// up rows); down 32 x 32 rows.
 template <int EPI>
 struct GemmShape {
     static constexpr int K = EPI == EPI_O ? kFQ : EPI == EPI_DOWN ? kFI : kFH;
-    static constexpr int NT = (EPI == EPI_QKV || EPI == EPI_GU) ? 8 : 4;
-    static constexpr int NRT = EPI == EPI_QKV ? 32 : EPI == EPI_GU ? 48 : 16;
+    static constexpr int ROWS = EPI == EPI_QKV ? 128 : EPI == EPI_O ? 64 : EPI == EPI_GU ? 96 : 32;
+    static constexpr int NT = ROWS / 16;
+    static constexpr int NRT = EPI == EPI_QKV ? 32 : EPI == EPI_O ? 16 : EPI == EPI_GU ? 64 : 32;
+    static_assert(ROWS * K <= kWtBytes, "row tile in LDS");
 };
+// K blocks whose A operands are in flight (NP = 4 with 8 spills)
+constexpr int pf_ring(int np) { return np == 4 ? 4 : 8; }
+constexpr int kGuCh = 48;                   // gate|up channels per row tile
 
+// Row tile rt's weights straight into LDS (no registers held), issued by waves 1-3 (wave 0 is
+// polling the grid barrier); the next grid barrier completes them. One instruction takes 8 rows x 128 bytes, whole lines, lane l the 16-byte chunk
+// (l % 8) ^ (l / 8) of row l / 8: its 1 KB block in LDS then holds chunk c of row r at slot
+// 8 r + (c ^ r), so that the 8 rows a quarter of a B operand's read touches lie in different banks.
 template <int EPI>
-__device__ void pf_gemm(const PfArgs& a, int tile, PfShared& sh) {
+__device__ __forceinline__ void pf_load_weights(const PfArgs& a, int layer, int rt, PfShared& sh) {
     using GS = GemmShape<EPI>;
-    constexpr int K = GS::K, NT = GS::NT, NK = K / 64;
+    constexpr int RG = GS::ROWS / 8, KC = GS::K / 128;
+    const int lane = pf_fresh(threadIdx.x) % kWave;
+    const int w = __builtin_amdgcn_readfirstlane(pf_fresh(threadIdx.x) / kWave);
+    if (w == 0) return;
+    // the tile's first row; gate|up: the gate rows', and the up rows' less the gate rows before them
+    const LayerWeights* const lw = a.lw + layer;
+    const int8_t* base;
+    const int8_t* base_up = nullptr;
+    if constexpr (EPI == EPI_QKV) {
+        const void *q = lw->q_proj_weight, *k = lw->k_proj_weight, *v = lw->v_proj_weight;
+        base = static_cast<const int8_t*>(rt < 16 ? q : rt < 24 ? k : v) + (size_t)128 * (rt < 16 ? rt : rt % 8) * GS::K;
+    } else if constexpr (EPI == EPI_GU) {
+        base = static_cast<const int8_t*>(lw->gate_proj_weight) + (size_t)kGuCh * rt * GS::K;
+        base_up = static_cast<const int8_t*>(lw->up_proj_weight) + ((int64_t)kGuCh * rt - kGuCh) * GS::K;
+    } else {
+        base = static_cast<const int8_t*>(EPI == EPI_O ? lw->o_proj_weight : lw->down_proj_weight) +
+               (size_t)GS::ROWS * rt * GS::K;
+    }
+    const size_t off = (size_t)(lane / 8) * GS::K + 16 * ((lane % 8) ^ (lane / 8));
+    for (int i = w - 1; i < RG * KC; i += 3) {
+        const int g = i / KC, kc = i % KC;
+        const int8_t* const rows = (EPI == EPI_GU && g >= kGuCh / 8 ? base_up : base) + (size_t)8 * g * GS::K;
+        __builtin_amdgcn_global_load_lds(
+            (const void __attribute__((address_space(1)))*)(rows + off + 128 * kc),
+            (void __attribute__((address_space(3)))*)(&sh.wt[(kc * RG + g) * kWave]), 16, 0, 0);
+    }
+}
+
+template <int EPI, int NP>
+__device__ void pf_gemm(const PfArgs& a, int rt, int pt, PfShared& sh) {
+    using GS = GemmShape<EPI>;
+    constexpr int K = GS::K, NT = GS::NT, NK = K / 64, RG = GS::ROWS / 8, D = pf_ring(NP);
+    static_assert(NK % D == 0 && D % 2 == 0, "whole rings");
     const PfLayout L = pf_layout((size_t)a.Pp);
     const int tid = pf_fresh(threadIdx.x), lane = tid % kWave, w = tid / kWave;
-    const int rt = tile % GS::NRT, pt = tile / GS::NRT;
-    const int p0 = kTileP * pt + 8 * w;
-    const int l16 = lane % 16;
+    const int p0 = 8 * NP * pt + 2 * NP * w;
+    const int l16 = lane % 16, kq = lane / 16;
     const LayerWeights lw = a.lw[a.layer];
     const ScalePointers sp = a.sp[a.layer];
 
-    // the lane's weight row of each block, and its scale
-    const int8_t* wrow[NT];
-    const float* srow[NT];
+    const float* srow[NT];                  // the lane's row scale of each block
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        const int8_t* base;
-        const float* sc;
-        int row;
-        if constexpr (EPI == EPI_QKV) {
-            if (rt < 16) { base = (const int8_t*)lw.q_proj_weight; sc = sp.q_scale; row = 128 * rt; }
-            else if (rt < 24) { base = (const int8_t*)lw.k_proj_weight; sc = sp.k_scale; row = 128 * (rt - 16); }
-            else { base = (const int8_t*)lw.v_proj_weight; sc = sp.v_scale; row = 128 * (rt - 24); }
-            row += 16 * t + l16;
-        } else if constexpr (EPI == EPI_GU) {
-            base = (const int8_t*)(t < 4 ? lw.gate_proj_weight : lw.up_proj_weight);
-            sc = t < 4 ? sp.gate_scale : sp.up_scale;
-            row = 64 * rt + 16 * (t % 4) + l16;
-        } else {
-            base = (const int8_t*)(EPI == EPI_O ? lw.o_proj_weight : lw.down_proj_weight);
-            sc = EPI == EPI_O ? sp.o_scale : sp.down_scale;
-            row = 64 * rt + 16 * t + l16;
-        }
-        wrow[t] = base + (size_t)row * K + 16 * (lane / 16);
-        srow[t] = sc + row;
+        if constexpr (EPI == EPI_QKV)
+            srow[t] = (rt < 16 ? sp.q_scale + 128 * rt : rt < 24 ? sp.k_scale + 128 * (rt - 16) : sp.v_scale + 128 * (rt - 24)) +
+                      16 * t + l16;
+        else if constexpr (EPI == EPI_GU)
+            srow[t] = (t < NT / 2 ? sp.gate_scale : sp.up_scale) + kGuCh * rt + 16 * (t % (NT / 2)) + l16;
+        else
+            srow[t] = (EPI == EPI_O ? sp.o_scale : sp.down_scale) + GS::ROWS * rt + 16 * t + l16;
     }
-    const uint8_t* abase = pf_buf<uint8_t>(a, L.dig) + (size_t)p0 * 512 + l16 * 64 + 16 * (lane / 16);
+    const uint8_t* abase = pf_buf<uint8_t>(a, L.dig) + (size_t)p0 * 512 + l16 * 64 + 16 * kq;
     const size_t kstride = (size_t)a.Pp * 512;
 
-    i32x4_t acc[4][NT];
+    i32x4_t A[D][NP];
+    auto load = [&](int d) {                // the next K block's A operands into stage d
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[j][t] = i32x4_t{0, 0, 0, 0};
-    // Each wave loads a quarter of a K block's weight tile (NB of the NT row blocks) and
-    // shares it through LDS: the four waves would otherwise each load the whole tile, and
-    // those loads (16 rows x 64 bytes per instruction) were most of a product's time.
-    constexpr int NB = NT / 4;
-    auto load = [&](int kb, i32x4_t (&A)[4], uint4 (&Bs)[NB]) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint4 u = ldg16(abase + kb * kstride + 1024 * j);
-            A[j] = i32x4_t{(int)u.x, (int)u.y, (int)u.z, (int)u.w};
+        for (int j = 0; j < NP; ++j) {
+            const uint4 u = ldg16(abase + 1024 * j);
+            A[d][j] = i32x4_t{(int)u.x, (int)u.y, (int)u.z, (int)u.w};
         }
-#pragma unroll
-        for (int u = 0; u < NB; ++u) Bs[u] = ldg16(wrow[NB * w + u] + 64 * kb);
+        abase += kstride;
     };
-    // three K blocks' operands in registers (stage kb % 3): block kb + 3's loads go into the
-    // registers block kb has just used, so each load has three blocks of work to arrive in
-    i32x4_t A0[4], A1[4], A2[4];
-    uint4 B0[NB], B1[NB], B2[NB];
-    load(0, A0, B0);
-    __builtin_amdgcn_sched_barrier(0);
-    if (NK > 1) load(1, A1, B1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (NK > 2) load(2, A2, B2);
-    __builtin_amdgcn_sched_barrier(0);
-    auto step = [&](int kb, i32x4_t (&A)[4], uint4 (&Bs)[NB]) {
-        // the wave's share into LDS buffer kb % 2; after the barrier every wave has finished
-        // block kb - 1, whose buffer kb + 1 will overwrite
-        uint4 (*gb)[kWave] = sh.gb[kb % 2];
 #pragma unroll
-        for (int u = 0; u < NB; ++u) gb[NB * w + u][lane] = Bs[u];
-        __syncthreads();
-        i32x4_t B[NT];
+    for (int d = 0; d < D; ++d) load(d);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // B operand t of K block kb: row 16 t + l16, chunk kq + 4 (kb % 2) of 128-byte column kb / 2
+    const uint4* const brow = &sh.wt[kWave * (l16 / 8) + 8 * (l16 % 8)];
+    const int ch[2] = {kq ^ (l16 % 8), (kq + 4) ^ (l16 % 8)};
+    i32x4_t B[2][NT];
+    auto readb = [&](int kb, int odd) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const uint4 u = gb[t][lane];
-            B[t] = i32x4_t{(int)u.x, (int)u.y, (int)u.z, (int)u.w};
+            const uint4 u = brow[kWave * ((kb / 2) * RG + 2 * t) + ch[odd]];
+            B[odd][t] = i32x4_t{(int)u.x, (int)u.y, (int)u.z, (int)u.w};
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int t = 0; t < NT; ++t) acc[j][t] = mfma_i8(A[j], B[t], acc[j][t]);
-        if (kb + 3 < NK) load(kb + 3, A, Bs);
-        // kept in this order: left to itself the scheduler moves later blocks' MFMAs up to
-        // the loads and waits for nearly every load in flight before the first of them
-        __builtin_amdgcn_sched_barrier(0);
     };
-    for (int kb = 0; kb < NK; kb += 3) {
-        step(kb, A0, B0);
-        if (kb + 1 < NK) step(kb + 1, A1, B1);
-        if (kb + 2 < NK) step(kb + 2, A2, B2);
+    i32x4_t acc[NP][NT];
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[j][t] = i32x4_t{0, 0, 0, 0};
+    readb(0, 0);
+    for (int kb0 = 0; kb0 < NK; kb0 += D) {
+        const bool more = kb0 + D < NK;     // uniform
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const int kb = kb0 + d;
+            if (d + 1 < D || more) readb(kb + 1, (d + 1) % 2);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NP; ++j)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[j][t] = mfma_i8(A[d][j], B[d % 2][t], acc[j][t]);
+            if (more) load(d);
+            // kept in this order: left to itself the scheduler moves later blocks' MFMAs up to
+            // the loads and waits for nearly every load in flight before the first of them
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
-    __syncthreads();                        // the last blocks' buffers are read before the next tile writes them
 
     // ---- epilogue ----
-    // Every global value the epilogue reads is requested first, for all four pairs, so that
+    // Every global value the epilogue reads is requested first, for all pairs, so that
     // they come back in one memory round trip (issued pair by pair, each pair waited for
-    // its own: four round trips per tile).
+    // its own: NP round trips per tile).
     const bool owner = (lane & 16) == 0;       // after tile_value: lanes 0-15 (even pair member), 32-47 (odd)
     const uint32_t* emax = pf_buf<uint32_t>(a, L.emax);
-    int pj[4];
-    uint32_t exv[4];
+    int pj[NP];
+    uint32_t exv[NP];
     float scv[NT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NP; ++j) {
         pj[j] = p0 + 2 * j + (lane >> 5);                  // chunk position of this lane's values (< Pp)
         exv[j] = emax[pj[j]];
     }
@@ -357,8 +388,8 @@ __device__ void pf_gemm(const PfArgs& a, int tile, PfShared& sh) {
     for (int t = 0; t < NT; ++t) scv[t] = *srow[t];
     // QKV: QK-norm gains and the positions' RoPE rows (bf16, rows clamped into the table);
     // O / down: the residual rows
-    uint32_t gnv[8], cs[4][16];
-    float res[4][NT];
+    uint32_t gnv[8], cs[NP][16];
+    float res[NP][NT];
     if constexpr (EPI == EPI_QKV) {
         if (rt < 24) {
             const uint16_t* gn = static_cast<const uint16_t*>(rt < 16 ? lw.q_norm_weight : lw.k_norm_weight);
@@ -368,7 +399,7 @@ __device__ void pf_gemm(const PfArgs& a, int tile, PfShared& sh) {
                 gnv[t + 4] = gn[16 * t + l16 + 64];
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < NP; ++j) {
                 const int pos = min(a.pos0 + pj[j], a.S - 1);
                 const uint16_t* cr = a.cos_t + (size_t)pos * kFD;
                 const uint16_t* sr = a.sin_t + (size_t)pos * kFD;
@@ -384,16 +415,16 @@ __device__ void pf_gemm(const PfArgs& a, int tile, PfShared& sh) {
         }
     } else if constexpr (EPI == EPI_O || EPI == EPI_DOWN) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NP; ++j)
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const int n = 64 * rt + 16 * t + l16;
+                const int n = GS::ROWS * rt + 16 * t + l16;
                 if constexpr (EPI == EPI_O) res[j][t] = bf16_bits_to_f32(pf_buf<uint16_t>(a, L.hid)[(size_t)pj[j] * kFH + n]);
                 else res[j][t] = pf_buf<float>(a, L.x)[(size_t)pj[j] * kFH + n];
             }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NP; ++j) {
         const int p = pj[j];
         double val[NT];
 #pragma unroll
@@ -448,7 +479,7 @@ __device__ void pf_gemm(const PfArgs& a, int tile, PfShared& sh) {
                 float* x = pf_buf<float>(a, L.x) + (size_t)p * kFH;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    const int n = 64 * rt + 16 * t + l16;
+                    const int n = GS::ROWS * rt + 16 * t + l16;
                     x[n] = (float)(val[t] * (double)scv[t] + (double)res[j][t]);
                 }
             }
@@ -456,10 +487,10 @@ __device__ void pf_gemm(const PfArgs& a, int tile, PfShared& sh) {
             if (store) {
                 float* m = pf_buf<float>(a, L.m) + (size_t)p * kFI;
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
+                for (int t = 0; t < NT / 2; ++t) {
                     const double gs = val[t] * (double)scv[t];
-                    const double us = val[t + 4] * (double)scv[t + 4];
-                    m[64 * rt + 16 * t + l16] = (float)silu_mul(gs, us);
+                    const double us = val[t + NT / 2] * (double)scv[t + NT / 2];
+                    m[kGuCh * rt + 16 * t + l16] = (float)silu_mul(gs, us);
                 }
             }
         } else {
@@ -467,10 +498,54 @@ __device__ void pf_gemm(const PfArgs& a, int tile, PfShared& sh) {
                 uint16_t* hid = pf_buf<uint16_t>(a, L.hid) + (size_t)p * kFH;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    const int n = 64 * rt + 16 * t + l16;
+                    const int n = GS::ROWS * rt + 16 * t + l16;
                     hid[n] = (uint16_t)f32_to_bf16_bits((float)(val[t] * (double)scv[t] + (double)res[j][t]));
                 }
             }
+        }
+    }
+}
+
+// The product's share of workgroup g: one row tile (the one prefetched, rt = g % NRT) against
+// position tiles grp, grp + groups, ... With NRT a multiple of 8 the groups of a row tile lie on
+// one XCD, so its weights come from HBM once. A grid smaller than NRT takes its further row
+// tiles' weights inside the phase. Position tiles hold 32 positions or, when that leaves fewer
+// rounds' work per workgroup, 16: a 16-position tile takes about 3/5 of a 32-position one's time
+// (QKV 8.3 against 13.7 us, gate|up 6.2 against 9.6 us, one tile per workgroup).
+template <int EPI>
+__device__ __forceinline__ int pf_groups(int G) { return max(G / GemmShape<EPI>::NRT, 1); }
+
+template <int EPI>
+__device__ __forceinline__ bool pf_has_tile(const PfArgs& a, int G, int g) {
+    return g / GemmShape<EPI>::NRT < min(pf_groups<EPI>(G), (a.P + 15) / 16);
+}
+
+// Issue the loads of workgroup g's row tile of a layer's product.
+template <int EPI>
+__device__ __forceinline__ void pf_prefetch(const PfArgs& a, int layer, PfShared& sh) {
+    const int G = (int)gridDim.x, g = pf_fresh_uniform((int)blockIdx.x);
+    if (pf_has_tile<EPI>(a, G, g)) pf_load_weights<EPI>(a, layer, g % GemmShape<EPI>::NRT, sh);
+}
+
+template <int EPI>
+__device__ __forceinline__ void pf_product(const PfArgs& a, PfShared& sh) {
+    constexpr int NRT = GemmShape<EPI>::NRT;
+    const int G = (int)gridDim.x, g = pf_fresh_uniform((int)blockIdx.x);
+    if (!pf_has_tile<EPI>(a, G, g)) return;
+    const int groups = pf_groups<EPI>(G), grp = g / NRT;
+    const int n32 = (a.P + 31) / 32, n16 = (a.P + 15) / 16;
+    const bool small = 3 * ((n16 + groups - 1) / groups) < 5 * ((n32 + groups - 1) / groups);
+    for (int rt = g % NRT; rt < NRT; rt += G) {
+        if (rt >= G) {                      // not the prefetched tile (uniform)
+            __syncthreads();
+            pf_load_weights<EPI>(a, a.layer, rt, sh);
+            wait_vmem();
+            __syncthreads();
+        }
+        if (small) {
+            for (int pt = grp; pt < n16; pt += groups) pf_gemm<EPI, 2>(a, rt, pt, sh);
+        } else {
+            for (int pt = grp; pt < n32; pt += groups) pf_gemm<EPI, 4>(a, rt, pt, sh);
         }
     }
 }
@@ -718,9 +793,16 @@ __device__ __forceinline__ bool pf_wait_ge(const uint32_t* p, uint32_t target, P
     return true;
 }
 
-__device__ __forceinline__ void pf_grid_barrier(PfSync* sy, uint32_t b, uint32_t limit) {
+//
+// `ahead` runs on waves 1-3 while wave 0 waits: it issues the loads of a coming product's weight
+// tile into LDS. The last workgroup barrier does not wait for them (lds_barrier: LDS
+// operations only); the next grid barrier does.
+template <class F>
+__device__ __forceinline__ void pf_grid_barrier(PfSync* sy, uint32_t b, uint32_t limit, F&& ahead) {
+    wait_vmem();                            // this wave's stores, and its loads into LDS
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) != 0) ahead();
+    else if (threadIdx.x == 0) {
         const uint32_t x = hw_xcc_id() % kPfXcd;
         const uint32_t per_xcd = gridDim.x / kPfXcd;
         const uint32_t old = __hip_atomic_fetch_add(&sy->xcd[x].arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -735,30 +817,31 @@ __device__ __forceinline__ void pf_grid_barrier(PfSync* sy, uint32_t b, uint32_t
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
     }
-    __syncthreads();
+    lds_barrier();
 }
 
-// The whole chunk in one launch: every layer's eight phases, each phase's work items dealt
-// over the workgroups: product tiles round-robin as rt + NRT pt (with NRT a multiple of 8 a
-// row tile's position tiles all run on one XCD and share its L2 copy of the weights),
-// attention items in units of even length (pf_attention_unit).
+// The whole chunk in one launch: every layer's nine phases, each phase's work items dealt
+// over the workgroups: positions round-robin, products as pf_product says, attention items in
+// units of even length (pf_attention_unit). A product's weights are requested two barriers
+// earlier, in the barrier before the digit phase of its input.
 __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
     __shared__ PfShared sh;
     const PfLayout L0 = pf_layout((size_t)a.Pp);
     PfSync* const sy = pf_buf<PfSync>(a, L0.sync);
     const int G = (int)gridDim.x, g = (int)blockIdx.x;
-    const int PT = (a.P + kTileP - 1) / kTileP;
     uint32_t nb = 0;
     int l = 0;
     auto stamp = [&](int point) {
         if (a.trace != nullptr && threadIdx.x == 0)
             a.trace[((size_t)l * kPfTracePoints + point) * G + g] = __builtin_amdgcn_s_memrealtime();
     };
-    auto barrier = [&](int k) {
+    auto barrier = [&](int k, auto&& ahead) {
         stamp(2 * k);
-        pf_grid_barrier(sy, ++nb, a.spin_limit);
+        pf_grid_barrier(sy, ++nb, a.spin_limit, ahead);
         stamp(2 * k + 1);
     };
+    auto none = [] {};
+    pf_prefetch<EPI_QKV>(a, 0, sh);
     for (l = 0; l < a.L; ++l) {
         PfArgs b = a;
         b.layer = l;
@@ -766,10 +849,10 @@ __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
             if (l == 0) pf_digits<kFH, SRC_EMBED>(b, p, sh);
             else pf_digits<kFH, SRC_HID>(b, p, sh);
         }
-        barrier(0);
-        for (int t = pf_fresh_uniform(g); t < GemmShape<EPI_QKV>::NRT * PT; t += G) pf_gemm<EPI_QKV>(b, t, sh);
+        barrier(0, none);
+        pf_product<EPI_QKV>(b, sh);
         if (l == a.L - 1) { stamp(2); break; }                 // the last layer contributes its cache rows only
-        barrier(1);
+        barrier(1, none);
         {
             // attention units, one per workgroup: a chunk of at most G items (KV head, tile of 8
             // positions) gives each workgroup one item; a longer one pairs tile j with tile
@@ -783,19 +866,19 @@ __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
                 pf_attention_unit(b, u % kFNKV, 8 * j, paired && jb > j ? 8 * jb : -1, sh);
             }
         }
-        barrier(2);
+        barrier(2, [&] { pf_prefetch<EPI_O>(a, l, sh); });
         for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFQ, SRC_A>(b, p, sh);
-        barrier(3);
-        for (int t = pf_fresh_uniform(g); t < GemmShape<EPI_O>::NRT * PT; t += G) pf_gemm<EPI_O>(b, t, sh);
-        barrier(4);
+        barrier(3, none);
+        pf_product<EPI_O>(b, sh);
+        barrier(4, [&] { pf_prefetch<EPI_GU>(a, l, sh); });
         for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFH, SRC_X>(b, p, sh);
-        barrier(5);
-        for (int t = pf_fresh_uniform(g); t < GemmShape<EPI_GU>::NRT * PT; t += G) pf_gemm<EPI_GU>(b, t, sh);
-        barrier(6);
+        barrier(5, none);
+        pf_product<EPI_GU>(b, sh);
+        barrier(6, [&] { pf_prefetch<EPI_DOWN>(a, l, sh); });
         for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFI, SRC_M>(b, p, sh);
-        barrier(7);
-        for (int t = pf_fresh_uniform(g); t < GemmShape<EPI_DOWN>::NRT * PT; t += G) pf_gemm<EPI_DOWN>(b, t, sh);
-        barrier(8);
+        barrier(7, none);
+        pf_product<EPI_DOWN>(b, sh);
+        barrier(8, [&] { pf_prefetch<EPI_QKV>(a, l + 1, sh); });
     }
 }
 

@@ -161,6 +161,20 @@ def test_chunked_prefill_equals_one_chunk(small):
     assert torch.equal(one[0], many[0]) and torch.equal(one[1], many[1])
 
 
+@pytest.mark.parametrize("P", [1, 15, 17, 33, 65, 129, 257, 300, 511])
+def test_prefill_position_tile_edges(small, P):
+    """One position either side of a product's 16- and 32-position tiles, and lengths at which the
+    products of a layer take different tile sizes or a ragged last round of tiles."""
+    dec, d, prompt, cfg, _ = small
+    ids = _tokens(P, cfg.vocab_size, 40 + P)
+    print(f"2-layer model: prefill of {P} positions vs {P} decode steps", flush=True)
+    _per_token(dec, ids)
+    want = _rows(dec, P)
+    dec.reset()
+    dec.prefill(ids)
+    _check_rows(_rows(dec, P), want, f"P={P}")
+
+
 def test_prefill_after_decode_steps(small):
     dec, d, prompt, cfg, _ = small
     ids = _tokens(45, cfg.vocab_size, 5)
