@@ -109,6 +109,9 @@ struct PfShared {
         double am[3][kWave][34];           // attention: parts handed to an item's leader wave (m, denominator, outputs)
         uint4 wt[kWtBytes / 16];           // products: the workgroup's weight rows, as pf_load_weights lays them out
     };
+    float sc[128];                         // their row scales
+    alignas(16) uint16_t qkg[kFD];                     // QKV: the QK-norm gains of the row tile's head
+    alignas(16) uint16_t gain[kFH];                    // RMSNorm gains of the next normed digit phase
     double reds[4];
     uint32_t rede[4];
 };
@@ -203,9 +206,9 @@ __device__ void pf_digits(const PfArgs& a, int p, PfShared& sh) {
         if (lane == 0) reds[wave] = ss;
         __syncthreads();
         const double rstd = rms_scale((reds[0] + reds[1]) + (reds[2] + reds[3]), K, kEps);
-        const LayerWeights lw = a.lw[a.layer];
-        const uint16_t* gain = static_cast<const uint16_t*>(SRC == SRC_X ? lw.post_attn_layernorm_weight
-                                                                         : lw.input_layernorm_weight);
+        // the gains were loaded into LDS a phase ahead (pf_load_gain), but for the launch's first
+        const uint16_t* gain = sh.gain;
+        if constexpr (SRC == SRC_EMBED) gain = static_cast<const uint16_t*>(a.lw[a.layer].input_layernorm_weight);
         const uint2 gu = *reinterpret_cast<const uint2*>(gain + 4 * t);
         const float gv[4] = {bf16_bits_to_f32(gu.x & 0xffffu), bf16_bits_to_f32(gu.x >> 16),
                              bf16_bits_to_f32(gu.y & 0xffffu), bf16_bits_to_f32(gu.y >> 16)};
@@ -234,9 +237,14 @@ __device__ void pf_digits(const PfArgs& a, int p, PfShared& sh) {
 // it against position tiles of 8 NP positions (32 or 16): wave w takes positions [8 NP pt +
 // 2 NP w, +2 NP) (NP pairs). Per 64-element K block a wave reads NT B operands (16 weight rows x
 // 64 bytes) from LDS and issues NP NT MFMAs on its NP A operands (a pair's 8 + 8 digit planes:
-// 1 KB contiguous), which are loaded pf_ring(NP) blocks ahead. The output tile of pair j, block t:
-// lane l (bit 4 clear) ends with the value of position 2j + l / 32 and weight row 16 t + l % 16
-// (tile_value).
+// 1 KB contiguous), which are loaded pf_ring(NP) blocks ahead. Lane n of a block's B operand takes
+// tile row pf_row(t, n), so that a lane ends with contiguous rows: 4 of them in each half of a
+// head (QKV: the RoPE pairs (i, i + 64) meet in the lane), 4 of O, 3 gate and the same 3 up
+// channels, 2 of down. Its values are those of position 2 (2u + h) + l / 32 for pairs (2u, 2u + 1),
+// h = bit 4 of l (pair_values). What the epilogue reads is requested before the K loop (residuals,
+// RoPE rows) or lies in LDS with the weights (scales, gains). With rows 16 apart in a lane (2-byte
+// loads and stores), half of the lanes idle and those reads after the loop, the phases at 512
+// positions took QKV 23.6, O 12.7, gate|up 30.7, down 25.9 us; now 16.2, 12.0, 23.6, 24.3.
 //
 // The weights do not depend on the phases before the product, so their loads are issued while
 // the workgroup waits in an earlier grid barrier (pf_load_weights) and cost the product nothing.
@@ -254,6 +262,7 @@ struct GemmShape {
     static constexpr int K = EPI == EPI_O ? kFQ : EPI == EPI_DOWN ? kFI : kFH;
     static constexpr int ROWS = EPI == EPI_QKV ? 128 : EPI == EPI_O ? 64 : EPI == EPI_GU ? 96 : 32;
     static constexpr int NT = ROWS / 16;
+    static constexpr int RPL = EPI == EPI_QKV || EPI == EPI_O ? 4 : EPI == EPI_GU ? 3 : 2;   // contiguous rows of a lane
     static constexpr int NRT = EPI == EPI_QKV ? 32 : EPI == EPI_O ? 16 : EPI == EPI_GU ? 64 : 32;
     static_assert(ROWS * K <= kWtBytes, "row tile in LDS");
 };
@@ -261,10 +270,24 @@ struct GemmShape {
 constexpr int pf_ring(int np) { return np == 4 ? 4 : 8; }
 constexpr int kGuCh = 48;                   // gate|up channels per row tile
 
+// The tile row of block t, lane n.
+template <int EPI>
+__device__ __forceinline__ int pf_row(int t, int n) {
+    constexpr int RPL = GemmShape<EPI>::RPL;
+    return 16 * RPL * (t / RPL) + RPL * n + t % RPL;
+}
+
+// Bytes of 4 per lane straight into LDS: lane l's word at dst + 4 l.
+__device__ __forceinline__ void lds_load4(void* dst, const void* src) {
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                     (void __attribute__((address_space(3)))*)dst, 4, 0, 0);
+}
+
 // Row tile rt's weights straight into LDS (no registers held), issued by waves 1-3 (wave 0 is
-// polling the grid barrier); the next grid barrier completes them. One instruction takes 8 rows x 128 bytes, whole lines, lane l the 16-byte chunk
-// (l % 8) ^ (l / 8) of row l / 8: its 1 KB block in LDS then holds chunk c of row r at slot
-// 8 r + (c ^ r), so that the 8 rows a quarter of a B operand's read touches lie in different banks.
+// polling the grid barrier), and its scales and QK-norm gains, by wave 1; the next grid barrier
+// completes them. One instruction takes 8 rows x 128 bytes, whole lines: its 1 KB block in LDS
+// holds 16-byte chunk c of row r at slot 8 (r % 8) + (c ^ (r / RPL % 8)), so that the rows that
+// eight lanes of a B operand read (RPL apart) lie in different banks.
 template <int EPI>
 __device__ __forceinline__ void pf_load_weights(const PfArgs& a, int layer, int rt, PfShared& sh) {
     using GS = GemmShape<EPI>;
@@ -274,26 +297,82 @@ __device__ __forceinline__ void pf_load_weights(const PfArgs& a, int layer, int 
     if (w == 0) return;
     // the tile's first row; gate|up: the gate rows', and the up rows' less the gate rows before them
     const LayerWeights* const lw = a.lw + layer;
+    const ScalePointers* const sp = a.sp + layer;
     const int8_t* base;
     const int8_t* base_up = nullptr;
+    const float* sc;
+    const float* sc_up = nullptr;
     if constexpr (EPI == EPI_QKV) {
         const void *q = lw->q_proj_weight, *k = lw->k_proj_weight, *v = lw->v_proj_weight;
-        base = static_cast<const int8_t*>(rt < 16 ? q : rt < 24 ? k : v) + (size_t)128 * (rt < 16 ? rt : rt % 8) * GS::K;
+        const float *qs = sp->q_scale, *ks = sp->k_scale, *vs = sp->v_scale;
+        const int head = rt < 16 ? rt : rt % 8;
+        base = static_cast<const int8_t*>(rt < 16 ? q : rt < 24 ? k : v) + (size_t)128 * head * GS::K;
+        sc = (rt < 16 ? qs : rt < 24 ? ks : vs) + 128 * head;
+        if (w == 1 && rt < 24) {
+            const void *qg = lw->q_norm_weight, *kg = lw->k_norm_weight;
+            const uint16_t* const gains = static_cast<const uint16_t*>(rt < 16 ? qg : kg) + 2 * lane;
+            if ((reinterpret_cast<uintptr_t>(gains) & 2) == 0) {
+                lds_load4(sh.qkg, gains);
+            } else {                        // a gain vector at an odd element offset
+                sh.qkg[2 * lane] = gains[0];
+                sh.qkg[2 * lane + 1] = gains[1];
+            }
+        }
     } else if constexpr (EPI == EPI_GU) {
         base = static_cast<const int8_t*>(lw->gate_proj_weight) + (size_t)kGuCh * rt * GS::K;
         base_up = static_cast<const int8_t*>(lw->up_proj_weight) + ((int64_t)kGuCh * rt - kGuCh) * GS::K;
+        sc = sp->gate_scale + kGuCh * rt;
+        sc_up = sp->up_scale + (kGuCh * rt - kGuCh);
     } else {
         base = static_cast<const int8_t*>(EPI == EPI_O ? lw->o_proj_weight : lw->down_proj_weight) +
                (size_t)GS::ROWS * rt * GS::K;
+        sc = (EPI == EPI_O ? sp->o_scale : sp->down_scale) + GS::ROWS * rt;
     }
-    const size_t off = (size_t)(lane / 8) * GS::K + 16 * ((lane % 8) ^ (lane / 8));
+    if (w == 1) {
+#pragma unroll
+        for (int i = 0; i < GS::ROWS; i += kWave) {
+            const int r = min(i + lane, GS::ROWS - 1);
+            lds_load4(&sh.sc[i], (EPI == EPI_GU && r >= kGuCh ? sc_up : sc) + r);
+        }
+    }
+    const size_t off = (size_t)(lane / 8) * GS::K;
     for (int i = w - 1; i < RG * KC; i += 3) {
         const int g = i / KC, kc = i % KC;
+        const int chunk = (lane % 8) ^ (((8 * g + lane / 8) / GS::RPL) % 8);
         const int8_t* const rows = (EPI == EPI_GU && g >= kGuCh / 8 ? base_up : base) + (size_t)8 * g * GS::K;
         __builtin_amdgcn_global_load_lds(
-            (const void __attribute__((address_space(1)))*)(rows + off + 128 * kc),
+            (const void __attribute__((address_space(1)))*)(rows + off + 128 * kc + 16 * chunk),
             (void __attribute__((address_space(3)))*)(&sh.wt[(kc * RG + g) * kWave]), 16, 0, 0);
     }
+}
+
+// The RMSNorm gains of the digit phase after next into LDS, by wave 1 inside a grid barrier.
+__device__ __forceinline__ void pf_load_gain(const void* gain, PfShared& sh) {
+    const int lane = pf_fresh(threadIdx.x) % kWave;
+    if (__builtin_amdgcn_readfirstlane(pf_fresh(threadIdx.x) / kWave) != 1) return;
+#pragma unroll
+    for (int i = 0; i < kFH; i += 2 * kWave) lds_load4(&sh.gain[i], static_cast<const uint16_t*>(gain) + i + 2 * lane);
+}
+
+// The exact values of two position pairs' output tiles. Of pair j's tile lane n (< 16) of each
+// lane half holds digit sums 0-3 of row n and lane n + 16 sums 4-7 (sum_d S_d 2^(49 - 7d), each
+// half exact in fp64); one exchange of 16-lane rows gives lane n pair c0's two halves and lane
+// n + 16 pair c1's, so that every lane finishes a value.
+__device__ __forceinline__ double pair_values(i32x4_t c0, i32x4_t c1) {
+    auto half = [](i32x4_t c) {
+        return fma((double)c[0], 2097152.0, fma((double)c[1], 16384.0, fma((double)c[2], 128.0, (double)c[3])));
+    };
+    const double h0 = half(c0), h1 = half(c1);
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)__double2loint(h0), (uint32_t)__double2loint(h1), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)__double2hiint(h0), (uint32_t)__double2hiint(h1), false, false);
+    return fma(__hiloint2double((int)hi[0], (int)lo[0]), 268435456.0, __hiloint2double((int)hi[1], (int)lo[1]));
+}
+
+// Four bf16 values (8 bytes) at dst.
+__device__ __forceinline__ void store_bf16x4(uint16_t* dst, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(dst) =
+        make_uint2((uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16),
+                   (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16));
 }
 
 template <int EPI, int NP>
@@ -305,19 +384,30 @@ __device__ void pf_gemm(const PfArgs& a, int rt, int pt, PfShared& sh) {
     const int tid = pf_fresh(threadIdx.x), lane = tid % kWave, w = tid / kWave;
     const int p0 = 8 * NP * pt + 2 * NP * w;
     const int l16 = lane % 16, kq = lane / 16;
-    const LayerWeights lw = a.lw[a.layer];
-    const ScalePointers sp = a.sp[a.layer];
-
-    const float* srow[NT];                  // the lane's row scale of each block
+    // What the epilogue reads of this lane's positions, requested before the K loop
+    constexpr int NU = NP / 2;
+    const int h = (lane >> 4) & 1;
+    int pj[NU];
+    uint32_t exv[NU];
+    uint2 cs[NU][4];                        // QKV: RoPE rows (cos low, cos high, sin low, sin high half)
+    uint2 resh[NU];                         // O: residual (bf16)
+    float2 resx[NU];                        // down: residual (fp32)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        if constexpr (EPI == EPI_QKV)
-            srow[t] = (rt < 16 ? sp.q_scale + 128 * rt : rt < 24 ? sp.k_scale + 128 * (rt - 16) : sp.v_scale + 128 * (rt - 24)) +
-                      16 * t + l16;
-        else if constexpr (EPI == EPI_GU)
-            srow[t] = (t < NT / 2 ? sp.gate_scale : sp.up_scale) + kGuCh * rt + 16 * (t % (NT / 2)) + l16;
-        else
-            srow[t] = (EPI == EPI_O ? sp.o_scale : sp.down_scale) + GS::ROWS * rt + 16 * t + l16;
+    for (int u = 0; u < NU; ++u) {
+        pj[u] = p0 + 2 * (2 * u + h) + (lane >> 5);        // chunk position of this lane's values (< Pp)
+        exv[u] = pf_buf<uint32_t>(a, L.emax)[pj[u]];
+        if constexpr (EPI == EPI_QKV) {
+            const int64_t at = (int64_t)min(a.pos0 + pj[u], a.S - 1) * kFD + 4 * l16;    // clamped into the table
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                __builtin_memcpy(&cs[u][i], a.cos_t + at + 64 * i, 8);       // tables at any element offset
+                __builtin_memcpy(&cs[u][2 + i], a.sin_t + at + 64 * i, 8);
+            }
+        } else if constexpr (EPI == EPI_O) {
+            resh[u] = *reinterpret_cast<const uint2*>(pf_buf<uint16_t>(a, L.hid) + (size_t)pj[u] * kFH + 64 * rt + 4 * l16);
+        } else if constexpr (EPI == EPI_DOWN) {
+            resx[u] = *reinterpret_cast<const float2*>(pf_buf<float>(a, L.x) + (size_t)pj[u] * kFH + 32 * rt + 2 * l16);
+        }
     }
     const uint8_t* abase = pf_buf<uint8_t>(a, L.dig) + (size_t)p0 * 512 + l16 * 64 + 16 * kq;
     const size_t kstride = (size_t)a.Pp * 512;
@@ -335,14 +425,19 @@ __device__ void pf_gemm(const PfArgs& a, int rt, int pt, PfShared& sh) {
     for (int d = 0; d < D; ++d) load(d);
     __builtin_amdgcn_sched_barrier(0);
 
-    // B operand t of K block kb: row 16 t + l16, chunk kq + 4 (kb % 2) of 128-byte column kb / 2
-    const uint4* const brow = &sh.wt[kWave * (l16 / 8) + 8 * (l16 % 8)];
+    // B operand t of K block kb: row pf_row(t, l16), chunk kq + 4 (kb % 2) of 128-byte column kb / 2
+    int bat[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int r = pf_row<EPI>(t, l16);
+        bat[t] = kWave * (r / 8) + 8 * (r % 8);
+    }
     const int ch[2] = {kq ^ (l16 % 8), (kq + 4) ^ (l16 % 8)};
     i32x4_t B[2][NT];
     auto readb = [&](int kb, int odd) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const uint4 u = brow[kWave * ((kb / 2) * RG + 2 * t) + ch[odd]];
+            const uint4 u = sh.wt[kWave * RG * (kb / 2) + bat[t] + ch[odd]];
             B[odd][t] = i32x4_t{(int)u.x, (int)u.y, (int)u.z, (int)u.w};
         }
     };
@@ -371,136 +466,82 @@ __device__ void pf_gemm(const PfArgs& a, int rt, int pt, PfShared& sh) {
     }
 
     // ---- epilogue ----
-    // Every global value the epilogue reads is requested first, for all pairs, so that
-    // they come back in one memory round trip (issued pair by pair, each pair waited for
-    // its own: NP round trips per tile).
-    const bool owner = (lane & 16) == 0;       // after tile_value: lanes 0-15 (even pair member), 32-47 (odd)
-    const uint32_t* emax = pf_buf<uint32_t>(a, L.emax);
-    int pj[NP];
-    uint32_t exv[NP];
     float scv[NT];
 #pragma unroll
-    for (int j = 0; j < NP; ++j) {
-        pj[j] = p0 + 2 * j + (lane >> 5);                  // chunk position of this lane's values (< Pp)
-        exv[j] = emax[pj[j]];
-    }
+    for (int t = 0; t < NT; ++t) scv[t] = sh.sc[pf_row<EPI>(t, l16)];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) scv[t] = *srow[t];
-    // QKV: QK-norm gains and the positions' RoPE rows (bf16, rows clamped into the table);
-    // O / down: the residual rows
-    uint32_t gnv[8], cs[NP][16];
-    float res[NP][NT];
-    if constexpr (EPI == EPI_QKV) {
-        if (rt < 24) {
-            const uint16_t* gn = static_cast<const uint16_t*>(rt < 16 ? lw.q_norm_weight : lw.k_norm_weight);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                gnv[t] = gn[16 * t + l16];
-                gnv[t + 4] = gn[16 * t + l16 + 64];
-            }
-#pragma unroll
-            for (int j = 0; j < NP; ++j) {
-                const int pos = min(a.pos0 + pj[j], a.S - 1);
-                const uint16_t* cr = a.cos_t + (size_t)pos * kFD;
-                const uint16_t* sr = a.sin_t + (size_t)pos * kFD;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int i = 16 * t + l16;
-                    cs[j][t] = cr[i];
-                    cs[j][4 + t] = cr[i + 64];
-                    cs[j][8 + t] = sr[i];
-                    cs[j][12 + t] = sr[i + 64];
-                }
-            }
-        }
-    } else if constexpr (EPI == EPI_O || EPI == EPI_DOWN) {
-#pragma unroll
-        for (int j = 0; j < NP; ++j)
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const int n = GS::ROWS * rt + 16 * t + l16;
-                if constexpr (EPI == EPI_O) res[j][t] = bf16_bits_to_f32(pf_buf<uint16_t>(a, L.hid)[(size_t)pj[j] * kFH + n]);
-                else res[j][t] = pf_buf<float>(a, L.x)[(size_t)pj[j] * kFH + n];
-            }
-    }
-#pragma unroll
-    for (int j = 0; j < NP; ++j) {
-        const int p = pj[j];
+    for (int u = 0; u < NU; ++u) {
+        const int p = pj[u];
+        const int e = (int)exv[u] - 181;
         double val[NT];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) val[t] = tile_value(acc[j][t], exv[j]);
-        const bool store = owner && p < a.P;
-        const int pos = a.pos0 + p;
+        for (int t = 0; t < NT; ++t) val[t] = ldexp(pair_values(acc[2 * u][t], acc[2 * u + 1][t]), e) * (double)scv[t];
+        const bool store = p < a.P;
         if constexpr (EPI == EPI_QKV) {
+            const int64_t crow = (((int64_t)a.layer * kFNKV + rt % 8) * a.S + (a.pos0 + p)) * kFD;    // K or V cache row
             if (rt < 24) {
-                // q or k head: fp32 value, QK RMSNorm over the head's 128 dims (8 blocks in the
-                // lane, 16 lanes of the row), RoPE on the pairs (i, i + 64) = blocks (t, t + 4)
+                // q or k head: fp32 value, QK RMSNorm over the head's 128 dims (8 in the lane,
+                // 16 lanes), RoPE on the pairs (i, i + 64)
                 float y[8];
                 double ss = 0.0;
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
-                    y[t] = (float)(val[t] * (double)scv[t]);
+                    y[t] = (float)val[t];
                     ss = fma((double)y[t], (double)y[t], ss);
                 }
                 ss += partner64<1>(ss);
                 ss += partner64<2>(ss);
                 ss += partner64<4>(ss);
                 ss += partner64<8>(ss);
-                if (store) {
-                    const double rs = rms_scale(ss, kFD, kEps);
-                    const int64_t crow = rt < 16 ? 0 : (((int64_t)a.layer * kFNKV + (rt - 16)) * a.S + pos) * kFD;
-                    float* qrow = pf_buf<float>(a, L.q) + (size_t)p * kFQ + 128 * rt;
+                const double rs = rms_scale(ss, kFD, kEps);
+                const uint2 g0 = *reinterpret_cast<const uint2*>(&sh.qkg[4 * l16]);
+                const uint2 g1 = *reinterpret_cast<const uint2*>(&sh.qkg[64 + 4 * l16]);
+                auto half16 = [](uint2 v, int i) { return bf16_bits_to_f32(((i & 2 ? v.y : v.x) >> (16 * (i & 1))) & 0xffffu); };
+                float o0[4], o1[4];
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const int i = 16 * t + l16;
-                        const double y0 = (double)y[t] * rs * (double)bf16_bits_to_f32(gnv[t]);
-                        const double y1 = (double)y[t + 4] * rs * (double)bf16_bits_to_f32(gnv[t + 4]);
-                        const double cl = bf16_bits_to_f32(cs[j][t]), ch = bf16_bits_to_f32(cs[j][4 + t]);
-                        const double sl = bf16_bits_to_f32(cs[j][8 + t]), sh = bf16_bits_to_f32(cs[j][12 + t]);
-                        const float o0 = (float)(y0 * cl - y1 * sl);
-                        const float o1 = (float)(y0 * sh + y1 * ch);
-                        if (rt < 16) {
-                            qrow[i] = o0;
-                            qrow[i + 64] = o1;
-                        } else {
-                            a.kc[crow + i] = (uint16_t)f32_to_bf16_bits(o0);
-                            a.kc[crow + i + 64] = (uint16_t)f32_to_bf16_bits(o1);
-                        }
+                for (int t = 0; t < 4; ++t) {
+                    const double y0 = (double)y[t] * rs * (double)half16(g0, t);
+                    const double y1 = (double)y[t + 4] * rs * (double)half16(g1, t);
+                    const double cl = half16(cs[u][0], t), ch = half16(cs[u][1], t);
+                    const double sl = half16(cs[u][2], t), sh = half16(cs[u][3], t);
+                    o0[t] = (float)(y0 * cl - y1 * sl);
+                    o1[t] = (float)(y0 * sh + y1 * ch);
+                }
+                if (store) {
+                    if (rt < 16) {
+                        float* const qrow = pf_buf<float>(a, L.q) + (size_t)p * kFQ + 128 * rt + 4 * l16;
+                        *reinterpret_cast<float4*>(qrow) = make_float4(o0[0], o0[1], o0[2], o0[3]);
+                        *reinterpret_cast<float4*>(qrow + 64) = make_float4(o1[0], o1[1], o1[2], o1[3]);
+                    } else {
+                        store_bf16x4(a.kc + crow + 4 * l16, o0);
+                        store_bf16x4(a.kc + crow + 64 + 4 * l16, o1);
                     }
                 }
             } else if (store) {
-                const int64_t crow = (((int64_t)a.layer * kFNKV + (rt - 24)) * a.S + pos) * kFD;
-#pragma unroll
-                for (int t = 0; t < 8; ++t)
-                    a.vc[crow + 16 * t + l16] = (uint16_t)f32_to_bf16_bits((float)(val[t] * (double)scv[t]));
+                const float v0[4] = {(float)val[0], (float)val[1], (float)val[2], (float)val[3]};
+                const float v1[4] = {(float)val[4], (float)val[5], (float)val[6], (float)val[7]};
+                store_bf16x4(a.vc + crow + 4 * l16, v0);
+                store_bf16x4(a.vc + crow + 64 + 4 * l16, v1);
             }
         } else if constexpr (EPI == EPI_O) {
             if (store) {
-                float* x = pf_buf<float>(a, L.x) + (size_t)p * kFH;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const int n = GS::ROWS * rt + 16 * t + l16;
-                    x[n] = (float)(val[t] * (double)scv[t] + (double)res[j][t]);
-                }
+                const float r[4] = {bf16_bits_to_f32(resh[u].x & 0xffffu), bf16_bits_to_f32(resh[u].x >> 16),
+                                    bf16_bits_to_f32(resh[u].y & 0xffffu), bf16_bits_to_f32(resh[u].y >> 16)};
+                *reinterpret_cast<float4*>(pf_buf<float>(a, L.x) + (size_t)p * kFH + 64 * rt + 4 * l16) =
+                    make_float4((float)(val[0] + (double)r[0]), (float)(val[1] + (double)r[1]),
+                                (float)(val[2] + (double)r[2]), (float)(val[3] + (double)r[3]));
             }
         } else if constexpr (EPI == EPI_GU) {
             if (store) {
-                float* m = pf_buf<float>(a, L.m) + (size_t)p * kFI;
+                float* const m = pf_buf<float>(a, L.m) + (size_t)p * kFI + kGuCh * rt + 3 * l16;
 #pragma unroll
-                for (int t = 0; t < NT / 2; ++t) {
-                    const double gs = val[t] * (double)scv[t];
-                    const double us = val[t + NT / 2] * (double)scv[t + NT / 2];
-                    m[kGuCh * rt + 16 * t + l16] = (float)silu_mul(gs, us);
-                }
+                for (int t = 0; t < 3; ++t) m[t] = (float)silu_mul(val[t], val[t + 3]);
             }
         } else {
             if (store) {
-                uint16_t* hid = pf_buf<uint16_t>(a, L.hid) + (size_t)p * kFH;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const int n = GS::ROWS * rt + 16 * t + l16;
-                    hid[n] = (uint16_t)f32_to_bf16_bits((float)(val[t] * (double)scv[t] + (double)res[j][t]));
-                }
+                const uint32_t lo = f32_to_bf16_bits((float)(val[0] + (double)resx[u].x));
+                const uint32_t hi = f32_to_bf16_bits((float)(val[1] + (double)resx[u].y));
+                *reinterpret_cast<uint32_t*>(pf_buf<uint16_t>(a, L.hid) + (size_t)p * kFH + 32 * rt + 2 * l16) = lo | (hi << 16);
             }
         }
     }
@@ -868,7 +909,7 @@ __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
         }
         barrier(2, [&] { pf_prefetch<EPI_O>(a, l, sh); });
         for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFQ, SRC_A>(b, p, sh);
-        barrier(3, none);
+        barrier(3, [&] { pf_load_gain(a.lw[l].post_attn_layernorm_weight, sh); });
         pf_product<EPI_O>(b, sh);
         barrier(4, [&] { pf_prefetch<EPI_GU>(a, l, sh); });
         for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFH, SRC_X>(b, p, sh);
@@ -876,7 +917,7 @@ __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
         pf_product<EPI_GU>(b, sh);
         barrier(6, [&] { pf_prefetch<EPI_DOWN>(a, l, sh); });
         for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFI, SRC_M>(b, p, sh);
-        barrier(7, none);
+        barrier(7, [&] { if (l + 1 < a.L) pf_load_gain(a.lw[l + 1].input_layernorm_weight, sh); });
         pf_product<EPI_DOWN>(b, sh);
         barrier(8, [&] { pf_prefetch<EPI_QKV>(a, l + 1, sh); });
     }
