@@ -87,18 +87,20 @@ struct PfArgs {
     uint64_t* trace;                       // optional phase timeline (kPfTracePoints per layer)
 };
 
-// Grid-barrier state. Counters are cumulative over a launch (zeroed before it), each on a
-// 64-byte line of its own.
+// Grid-barrier state. Counters are cumulative over a launch (zeroed before it); each XCD has a
+// 128-byte cache line of its own.
 constexpr int kPfXcd = 8;
 constexpr int kPfTracePoints = 18;            // phase k (9 per layer): 2 k phase done, 2 k + 1 barrier passed
 struct PfSync {
-    uint32_t count;                        // XCD leaders that reached the current barrier
-    uint32_t abort;                        // set when a barrier wait expired
-    uint32_t pad0[14];
     struct {
         uint32_t arrived;                  // workgroups of the XCD that reached the current barrier
+        uint32_t pad0[7];
         uint32_t released;                 // the last barrier the XCD's leader has passed
-        uint32_t pad[14];
+        uint32_t pad1[7];
+        uint32_t lead;                     // the last barrier the XCD's leader has reached
+        uint32_t pad2[7];
+        uint32_t abort;                    // xcd[0]'s: set when a barrier wait expired
+        uint32_t pad3[7];
     } xcd[kPfXcd];
 };
 static_assert(sizeof(PfSync) <= 1024, "barrier state");
@@ -811,30 +813,36 @@ __device__ void pf_attention_unit(const PfArgs& a, int x, int pa, int pb, PfShar
 }
 
 // ---- grid barrier ----------------------------------------------------------------------
-// Two levels. A workgroup's results are in its XCD's L2 once it reaches the barrier (the
-// workgroup barrier first waits for its stores). The last workgroup of an XCD to arrive is
-// that XCD's leader: its agent-scope release writes the XCD's L2 back to memory (once per XCD
-// and barrier: one write-back per workgroup, 32 per XCD, cost 26-90 us per barrier), then it
-// arrives at the grid counter, waits for the other seven leaders, drops stale lines of the
-// L2 (acquire) and releases its XCD's workgroups, which drop their own stale lines. Barrier
-// number b completes when the counters reach b times their arrivals. A wait that expires
-// sets the abort flag, and every later wait of the launch then returns at once, so the
-// grid always drains (the host reports MQ_ERR_TIMEOUT, mq_prefill_check). Needs the
+// Two levels. A workgroup's results are in its XCD's L2 once it reaches the barrier (each wave
+// waits for its own stores first). The last workgroup of an XCD to arrive, counted by an atomic
+// that the XCD's L2 performs, is that XCD's leader: its agent-scope release writes the XCD's L2
+// back to memory (once per XCD and barrier: one write-back per workgroup, 32 per XCD, cost 26-90
+// us per barrier), then it raises its flag, waits for all eight leaders' flags (eight lanes, one
+// flag each), drops the L2's stale lines, waits for that, and releases its XCD's workgroups through
+// the L2. These drop the stale lines of their own L1 only: every XCD had written its results back
+// before the L2 was cleared, and nothing but weights is read in between. (An agent-scope acquire
+// in every workgroup clears the L2 32 times, the later ones under the phase that has begun: each
+// phase took about 1.3 us longer, a layer 89 instead of 79 us at 77 positions, 173 instead of
+// 165 at 512.) Barrier number b
+// completes when an XCD's arrivals reach b times its workgroups and the flags reach b. A wait
+// that expires sets the abort flag, and every later wait of the launch then returns at once,
+// so the grid always drains (the host reports MQ_ERR_TIMEOUT, mq_prefill_check). Needs the
 // workgroups dealt round-robin over the 8 XCDs (checked by the host).
+//
+// Waits until every active lane's word has reached the target; runs on a whole wave.
 __device__ __forceinline__ bool pf_wait_ge(const uint32_t* p, uint32_t target, PfSync* sy, uint32_t limit) {
     uint32_t n = 0;
-    while (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-        if (__hip_atomic_load(&sy->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return false;
-        __builtin_amdgcn_s_sleep(2);
+    while (__any(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)) {
+        if (__hip_atomic_load(&sy->xcd[0].abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return false;
+        __builtin_amdgcn_s_sleep(1);
         if (++n >= limit) {
-            __hip_atomic_store(&sy->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&sy->xcd[0].abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return false;
         }
     }
     return true;
 }
 
-//
 // `ahead` runs on waves 1-3 while wave 0 waits: it issues the loads of a coming product's weight
 // tile into LDS. The last workgroup barrier does not wait for them (lds_barrier: LDS
 // operations only); the next grid barrier does.
@@ -842,20 +850,23 @@ template <class F>
 __device__ __forceinline__ void pf_grid_barrier(PfSync* sy, uint32_t b, uint32_t limit, F&& ahead) {
     wait_vmem();                            // this wave's stores, and its loads into LDS
     __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) != 0) ahead();
-    else if (threadIdx.x == 0) {
-        const uint32_t x = hw_xcc_id() % kPfXcd;
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) != 0) {
+        ahead();
+    } else {
+        const int lane = threadIdx.x % kWave;
+        auto& mine = sy->xcd[hw_xcc_id() % kPfXcd];
         const uint32_t per_xcd = gridDim.x / kPfXcd;
-        const uint32_t old = __hip_atomic_fetch_add(&sy->xcd[x].arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (old == b * per_xcd - 1u) {
+        uint32_t old = 0;
+        if (lane == 0) old = __hip_atomic_fetch_add(&mine.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)old) == b * per_xcd - 1u) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            __hip_atomic_fetch_add(&sy->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            pf_wait_ge(&sy->count, b * kPfXcd, sy, limit);
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            __hip_atomic_store(&sy->xcd[x].released, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (lane == 0) __hip_atomic_store(&mine.lead, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            pf_wait_ge(&sy->xcd[lane % kPfXcd].lead, b, sy, limit);
+            asm volatile("buffer_inv sc1\n\ts_waitcnt vmcnt(0)" ::: "memory");      // this XCD's L2, this CU's L1: done
+            if (lane == 0) __hip_atomic_store(&mine.released, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         } else {
-            pf_wait_ge(&sy->xcd[x].released, b, sy, limit);
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            pf_wait_ge(&mine.released, b, sy, limit);
+            asm volatile("buffer_inv sc0\n\ts_waitcnt vmcnt(0)" ::: "memory");      // this CU's L1
         }
     }
     lds_barrier();
@@ -924,15 +935,15 @@ __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
 }
 
 __global__ void pf_sync_reset_kernel(PfSync* sy) {
-    sy->count = 0u;
-    sy->abort = 0u;
+    sy->xcd[0].abort = 0u;
     for (int x = 0; x < kPfXcd; ++x) {
         sy->xcd[x].arrived = 0u;
         sy->xcd[x].released = 0u;
+        sy->xcd[x].lead = 0u;
     }
 }
 
-__global__ void pf_sync_status_kernel(const PfSync* sy, uint32_t* out) { *out = sy->abort; }
+__global__ void pf_sync_status_kernel(const PfSync* sy, uint32_t* out) { *out = sy->xcd[0].abort; }
 
 }  // namespace
 
