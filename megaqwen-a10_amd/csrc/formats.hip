@@ -17,6 +17,7 @@
 #include "common.h"
 #include "digits.h"
 #include "internal.h"
+#include "quant_rows.h"
 
 #include <algorithm>
 
@@ -28,18 +29,7 @@ constexpr int kFmtThreads = 256;
 constexpr int kFmtWaves = kFmtThreads / kWave;
 constexpr int kInt4Group = 128;
 
-// ---- quantizers ------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t fp8_e4m3_encode(float x) {
-    const uint32_t sign = (__float_as_uint(x) >> 24) & 0x80u;
-    const float a = fabsf(x);
-    if (!(a < 448.0f)) return sign | 0x7Eu;                       // saturate (and NaN)
-    if (a < 0x1p-6f) return sign | (uint32_t)__builtin_rintf(a * 512.0f);   // subnormal: m 2^-9, exact scaling
-    const uint32_t u = __float_as_uint(a);
-    const uint32_t r = (u + 0x7FFFFu + ((u >> 20) & 1u)) & 0xFFF00000u;      // mantissa to 3 bits, RNE
-    const int e = (int)(r >> 23) - 127;
-    return sign | ((uint32_t)(e + 7) << 3) | ((r >> 20) & 7u);
-}
-
+// ---- quantizers: rows that quant_rows.h does not take (odd lengths, unaligned views) --------
 __device__ __forceinline__ float block_max_abs(float v, float* red) {
     v = wave_max(v);
     const int wave = threadIdx.x / kWave;
@@ -169,25 +159,13 @@ fp8_gemv_kernel(const float* __restrict__ x, const uint8_t* __restrict__ w, int6
     }
 }
 
-int device_cus() {
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
-
 template <int R, int CHMAX>
 int launch_fp8_t(const float* x, const uint8_t* w, int64_t copy_stride, int n_copies, const float* scale, float* y,
                  int M, int K, int reps, hipStream_t stream) {
     constexpr int P = 16;
     const int64_t items = (int64_t)reps * ((M + R - 1) / R);
     const int64_t want = (items + kFmtWaves - 1) / kFmtWaves;
-    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(want, 8 * device_cus()));
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(want, 8 * device_cu_count()));
     const int CH = (K + 64 * P - 1) / (64 * P);
     const size_t lds = (size_t)CH * 64 * P * sizeof(float);
     hipLaunchKernelGGL((fp8_gemv_kernel<R, CHMAX>), dim3(grid), dim3(kFmtThreads), lds, stream,
@@ -199,7 +177,7 @@ int launch_fp8_t(const float* x, const uint8_t* w, int64_t copy_stride, int n_co
 // gives every CU at least two workgroups of items.
 int fmt_rows_per_item(int M, int CH, int reps) {
     int R = CH <= 1 ? 8 : CH == 2 ? 4 : CH <= 4 ? 2 : 1;
-    const int64_t min_waves = (int64_t)2 * kFmtWaves * device_cus();
+    const int64_t min_waves = (int64_t)2 * kFmtWaves * device_cu_count();
     while (R > 1 && (int64_t)reps * ((M + R - 1) / R) < min_waves) R /= 2;
     return R;
 }
@@ -367,7 +345,7 @@ int launch_int4_t(const float* x, const uint8_t* w, int64_t copy_stride, int n_c
                   int M, int K, int reps, hipStream_t stream) {
     const int64_t items = (int64_t)reps * ((M + 15) / 16);
     const int64_t want = (items + kFmtWaves - 1) / kFmtWaves;
-    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(want, 8 * device_cus()));
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(want, 8 * device_cu_count()));
     const size_t lds = (size_t)8 * (K + 16) + sizeof(double) * (K / kInt4Group);   // <= 132 KB (K <= 16384)
     if (lds > 65536) {
         static bool raised[64] = {false};          // per device: the limit is the current device's
@@ -389,12 +367,20 @@ int launch_int4_t(const float* x, const uint8_t* w, int64_t copy_stride, int n_c
 }  // namespace
 
 int launch_quantize_fp8(const void* w_bf16, int M, int K, uint8_t* q, float* scale, hipStream_t stream) {
+    if (quant_rows_fit(w_bf16, K, q, 8)) {
+        launch_quant_rows<Q_FP8>(w_bf16, M, K, q, scale, device_cu_count(), stream);
+        return check_launch("quantize_fp8");
+    }
     hipLaunchKernelGGL(quantize_fp8_rows_kernel, dim3(M), dim3(kFmtThreads), 0, stream,
                        static_cast<const uint16_t*>(w_bf16), (int64_t)K, q, scale);
     return check_launch("quantize_fp8_rows_kernel");
 }
 
 int launch_quantize_int4(const void* w_bf16, int M, int K, uint8_t* q, float* scale, hipStream_t stream) {
+    if (quant_rows_fit(w_bf16, K, q, 4)) {
+        launch_quant_rows<Q_INT4>(w_bf16, M, K, q, scale, device_cu_count(), stream);
+        return check_launch("quantize_int4");
+    }
     hipLaunchKernelGGL(quantize_int4_groups_kernel, dim3(M), dim3(kFmtThreads), 0, stream,
                        static_cast<const uint16_t*>(w_bf16), (int64_t)K, q, scale);
     return check_launch("quantize_int4_groups_kernel");

@@ -79,7 +79,7 @@ int8_gemv_kernel(const float* __restrict__ x, const int8_t* __restrict__ w, int6
     }
 }
 
-static int device_cu_count() {
+int device_cu_count() {
     static int cached[64] = {0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;

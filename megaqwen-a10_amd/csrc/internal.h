@@ -21,6 +21,7 @@ int launch_fp8_gemv(const float* x, const uint8_t* w, int64_t copy_stride, int n
                     int M, int K, int reps, hipStream_t stream);
 int launch_int4_gemv(const float* x, const uint8_t* w, int64_t copy_stride, int n_copies, const float* scale, float* y,
                      int M, int K, int reps, hipStream_t stream);
+int device_cu_count();          // compute units of the current device
 int launch_int8_gemv(const float* x, const int8_t* w, const float* scale, float* y, int M, int K,
                      hipStream_t stream);
 int launch_int8_gemv_repeat(const float* x, const int8_t* w, int64_t copy_stride, int n_copies, const float* scale,

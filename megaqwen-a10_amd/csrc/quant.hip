@@ -4,10 +4,12 @@
 //   scale = bf16_rne(amax / 127.0f)       the reference divides in bf16
 //           widened to fp32, clamped to >= 1e-12f
 //   q     = clamp(rint(fp32(w) / scale), -128, 127)   IEEE division, ties to even
-// One workgroup per row; each thread reads the row's bf16 elements k = tid, tid + 256, ...
-// (2-byte loads; the quantizer runs once at load time, off the decode path).
+// Rows of whole 16-byte loads up to 8192 elements go through the row pass of quant_rows.h; the
+// kernel here takes the others (odd lengths, longer rows, unaligned views): one workgroup per
+// row, each thread reading the row's bf16 elements k = tid, tid + 256, ...
 #include "common.h"
 #include "internal.h"
+#include "quant_rows.h"
 
 namespace mq {
 
@@ -43,6 +45,10 @@ quantize_rows_kernel(const uint16_t* __restrict__ w, int64_t K, int8_t* __restri
 }
 
 int launch_quantize(const void* w_bf16, int M, int K, int8_t* q, float* scale, hipStream_t stream) {
+    if (quant_rows_fit(w_bf16, K, q, 8)) {
+        launch_quant_rows<Q_INT8>(w_bf16, M, K, reinterpret_cast<uint8_t*>(q), scale, device_cu_count(), stream);
+        return check_launch("quantize_rows_wave_kernel");
+    }
     hipLaunchKernelGGL(quantize_rows_kernel, dim3(M), dim3(kQuantThreads), 0, stream,
                        static_cast<const uint16_t*>(w_bf16), (int64_t)K, q, scale);
     return check_launch("quantize_rows_kernel");
