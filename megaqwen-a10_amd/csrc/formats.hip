@@ -7,15 +7,14 @@
 //   INT4 per group of 128 elements of a row: s = bf16(amax / 7), q = clamp(rint(w / s), -8, 7),
 //        two's complement nibbles, low nibble = even element
 // Matvecs y[j] = sum_k dequant(w)[j, k] x[k], fp32 x and y.
-//   FP8: the structure of the INT8 matvec (one 16-byte load per lane per 1 KB of a row, the
-//        activation in LDS in per-lane order, R rows per wave item, the same steady-state
-//        repeat form), 16 weights per lane per load, 8 v_cvt_pk_f32_fp8, fp32 accumulation,
-//        the row scale applied after the row sum.
+//   FP8: the row kernel of gemv_rows.h, as the INT8 matvec: 8 v_cvt_pk_f32_fp8 per 16 weights,
+//        fp32 accumulation, the row scale applied after the row sum.
 //   INT4: on the int8 matrix cores, as the decode step's products: x as a 55-bit fixed-point
 //        vector in eight digit planes, the biased nibbles as the int8 operand, exact integer
 //        sums per group of 128, recombined and scaled in fp64 (int4_gemv_kernel).
 #include "common.h"
 #include "digits.h"
+#include "gemv_rows.h"
 #include "internal.h"
 #include "quant_rows.h"
 
@@ -78,122 +77,6 @@ quantize_int4_groups_kernel(const uint16_t* __restrict__ w, int64_t K, uint8_t* 
 }
 
 // ---- matvecs -----------------------------------------------------------------------------
-// P weights per lane per 16-byte load (16 FP8 codes).
-template <int P>
-__device__ __forceinline__ int fmt_xs_index(int k) {              // float index of element k
-    const int chunk = k / (64 * P);
-    const int e = k % (64 * P);
-    const int lane = e / P;
-    const int t = e % P;
-    return ((chunk * (P / 4) + (t >> 2)) * 64 + lane) * 4 + (t & 3);
-}
-
-// 16 FP8 codes against 16 activations (x[i] holds elements 4i .. 4i + 3)
-__device__ __forceinline__ float dot_fp8x16_regs(uint4 w, const float4 (&x)[4], float acc) {
-    const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float4 xv = x[i];
-        const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[i], false);   // bytes 0, 1
-        const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)wv[i], true);    // bytes 2, 3
-        acc = fmaf(lo[0], xv.x, acc);
-        acc = fmaf(lo[1], xv.y, acc);
-        acc = fmaf(hi[0], xv.z, acc);
-        acc = fmaf(hi[1], xv.w, acc);
-    }
-    return acc;
-}
-
-// FP8 per row (scale [M]).
-template <int R, int CHMAX>
-__global__ void __launch_bounds__(kFmtThreads)
-fp8_gemv_kernel(const float* __restrict__ x, const uint8_t* __restrict__ w, int64_t copy_stride, int n_copies,
-                const float* __restrict__ scale, float* __restrict__ y, int M, int K, int reps) {
-    constexpr int P = 16;                            // weights per lane per 16-byte load
-    extern __shared__ float4 xs[];
-    const int CH = (K + 64 * P - 1) / (64 * P);
-    float* xsf = reinterpret_cast<float*>(xs);
-    for (int k = threadIdx.x; k < CH * 64 * P; k += kFmtThreads) xsf[fmt_xs_index<P>(k)] = (k < K) ? x[k] : 0.0f;
-    __syncthreads();
-
-    const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
-    const int total_waves = gridDim.x * kFmtWaves;
-    const int nbatch = (M + R - 1) / R;
-    const int items = reps * nbatch;                 // < 2^31, checked by the host
-
-    for (int it = blockIdx.x * kFmtWaves + wave; it < items; it += total_waves) {
-        const int rep = it / nbatch;
-        const int row0 = (it - rep * nbatch) * R;
-        const int copy = rep % n_copies;
-        const uint8_t* const wc = w + (int64_t)copy * copy_stride;
-        uint4 wv[R][CHMAX];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-#pragma unroll
-            for (int c = 0; c < CHMAX; ++c) {
-                wv[r][c] = make_uint4(0, 0, 0, 0);
-                const int col = c * 64 * P + lane * P;     // first element of the lane's piece
-                if (c < CH && row0 + r < M && col < K)
-                    wv[r][c] = *reinterpret_cast<const uint4*>(wc + (int64_t)(row0 + r) * K + col);
-            }
-        }
-        // chunk outer, rows inner: the lane's 16 activations of a chunk are read from LDS
-        // once and used for all R rows
-        float acc[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-#pragma unroll
-        for (int c = 0; c < CHMAX; ++c) {
-            if (c < CH) {
-                const float4* frag = xs + (c * (P / 4)) * 64 + lane;
-                const float4 xv[4] = {frag[0], frag[64], frag[128], frag[192]};
-#pragma unroll
-                for (int r = 0; r < R; ++r) acc[r] = dot_fp8x16_regs(wv[r][c], xv, acc[r]);
-            }
-        }
-        const float s = transpose_reduce<R>(acc, lane);
-        constexpr int span = kWave / R;
-        const int row = row0 + lane / span;
-        if ((lane % span) == 0 && row < M) y[(int64_t)copy * M + row] = s * scale[row];
-    }
-}
-
-template <int R, int CHMAX>
-int launch_fp8_t(const float* x, const uint8_t* w, int64_t copy_stride, int n_copies, const float* scale, float* y,
-                 int M, int K, int reps, hipStream_t stream) {
-    constexpr int P = 16;
-    const int64_t items = (int64_t)reps * ((M + R - 1) / R);
-    const int64_t want = (items + kFmtWaves - 1) / kFmtWaves;
-    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(want, 8 * device_cu_count()));
-    const int CH = (K + 64 * P - 1) / (64 * P);
-    const size_t lds = (size_t)CH * 64 * P * sizeof(float);
-    hipLaunchKernelGGL((fp8_gemv_kernel<R, CHMAX>), dim3(grid), dim3(kFmtThreads), lds, stream,
-                       x, w, copy_stride, n_copies, scale, y, M, K, reps);
-    return check_launch("fp8_gemv");
-}
-
-// Rows per wave item as in the INT8 matvec: the largest R for the row length that still
-// gives every CU at least two workgroups of items.
-int fmt_rows_per_item(int M, int CH, int reps) {
-    int R = CH <= 1 ? 8 : CH == 2 ? 4 : CH <= 4 ? 2 : 1;
-    const int64_t min_waves = (int64_t)2 * kFmtWaves * device_cu_count();
-    while (R > 1 && (int64_t)reps * ((M + R - 1) / R) < min_waves) R /= 2;
-    return R;
-}
-
-template <int CHMAX>
-int launch_fp8_r(int R, const float* x, const uint8_t* w, int64_t copy_stride, int n_copies, const float* scale,
-                 float* y, int M, int K, int reps, hipStream_t stream) {
-    constexpr int RMAX = CHMAX <= 1 ? 8 : CHMAX == 2 ? 4 : CHMAX <= 4 ? 2 : 1;
-#define MQ_FMT(RR)                                                                                      \
-    if constexpr (RR <= RMAX)                                                                           \
-        if (R == RR) return launch_fp8_t<RR, CHMAX>(x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
-    MQ_FMT(8) MQ_FMT(4) MQ_FMT(2)
-#undef MQ_FMT
-    return launch_fp8_t<1, CHMAX>(x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
-}
-
 // ---- INT4 matvec on the int8 matrix cores ----------------------------------------------------
 // y[j] = sum_g s[j, g] sum_{k in g} q[j, k] x[k], with the decode step's exact products: x
 // becomes X_k = trunc(x_k 2^(181 - emax)) (emax the largest biased exponent of x; |X_k| <
@@ -388,14 +271,7 @@ int launch_quantize_int4(const void* w_bf16, int M, int K, uint8_t* q, float* sc
 
 int launch_fp8_gemv(const float* x, const uint8_t* w, int64_t copy_stride, int n_copies, const float* scale, float* y,
                     int M, int K, int reps, hipStream_t stream) {
-    constexpr int P = 16;
-    const int CH = (K + 64 * P - 1) / (64 * P);
-    const int R = fmt_rows_per_item(M, CH, reps);
-    if (CH <= 1) return launch_fp8_r<1>(R, x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
-    if (CH == 2) return launch_fp8_r<2>(R, x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
-    if (CH <= 4) return launch_fp8_r<4>(R, x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
-    if (CH <= 8) return launch_fp8_r<8>(R, x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
-    return launch_fp8_r<16>(R, x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
+    return launch_gemv_rows<Fp8W>(x, w, copy_stride, n_copies, scale, y, M, K, reps, stream);
 }
 
 int launch_int4_gemv(const float* x, const uint8_t* w, int64_t copy_stride, int n_copies, const float* scale, float* y,
