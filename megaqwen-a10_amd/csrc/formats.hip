@@ -107,143 +107,227 @@ quantize_int4_groups_kernel(const uint16_t* __restrict__ w, int64_t K, uint8_t* 
 // use them: 16-byte loads of four groups' scales when K / 128 is a multiple of 4. (16 rows of
 // 64 bytes per load, and one 4-byte scale load per group, measured 0.50-0.56 of the HBM
 // peak at the Qwen3-0.6B shapes; this form 0.69-0.81.)
-constexpr int kW4Unroll = 8;                      // groups whose loads are issued together (even)
+//
+// Work. A workgroup takes tiles of 16 rows, each cut along K over S of its waves (whole pairs
+// of groups; S = 1 where there are tiles enough for eight waves a CU). The waves' fp64 partial
+// sums of a tile meet in LDS and are added in wave order. A wave requests its first tile's
+// weights before the workgroup forms the digit planes, eight consecutive elements per
+// thread. Without the cut, and with the planes formed first, byte by byte, from one element per
+// load, single calls took (us, kernel) [1024, 3072] 15.3, [2048, 6144] 29.9, [12288, 2048] 12.4,
+// [6144, 1024] 8.0, [151936, 1024] 28.2; now 6.9, 7.8, 10.2, 6.3 and 21.
+constexpr int kW4Unroll = 4;                      // group pairs whose loads are issued together
+constexpr int kW4MaxWaves = 16;
 
-__device__ __forceinline__ int int4_plane_byte(int k) {
-    const int r = k & 127, e = r & 15;
-    const int j = (e & 1) ? ((e < 8) ? 4 + (e >> 1) : 12 + ((e - 9) >> 1)) : ((e < 8) ? (e >> 1) : 8 + ((e - 8) >> 1));
-    return (k & ~127) + 64 * ((r >> 4) & 1) + 16 * (r >> 5) + j;
+// Byte of element k (k % 8 == 0) in a digit plane; elements k .. k + 7 follow it in the order
+// 0 2 4 6 1 3 5 7.
+__device__ __forceinline__ int int4_plane_byte8(int k) {
+    const int r = k & 127;
+    return (k & ~127) + 64 * ((r >> 4) & 1) + 16 * (r >> 5) + (r & 8);
 }
 
-__global__ void __launch_bounds__(kFmtThreads)
+// kCut: S > 1 and the first tile's weights requested first; otherwise workgroups of four waves, a
+// tile each, whose next loads overlap across the waves (the prefetch's registers would cost one
+// wave in five: [1024, 2048] in a stream of matvecs 0.179 -> 0.190 us).
+template <bool kCut>
+__global__ void __launch_bounds__(kCut ? kW4MaxWaves * kWave : kFmtThreads)
 int4_gemv_kernel(const float* __restrict__ x, const uint8_t* __restrict__ w, int64_t copy_stride, int n_copies,
-                 const float* __restrict__ scale, float* __restrict__ y, int M, int K, int reps, bool vec_scales) {
+                 const float* __restrict__ scale, float* __restrict__ y, int M, int K, int reps, int S, bool vec_scales) {
     extern __shared__ __align__(16) uint8_t w4lds[];
-    __shared__ uint32_t red[kFmtWaves];
+    __shared__ uint32_t red[kW4MaxWaves];
+    __shared__ double part[2][kW4MaxWaves][16];
     constexpr int U = kW4Unroll;
     const int PS = K + 16;                        // digit plane stride in bytes
     uint8_t* const planes = w4lds;
     double* const sg = reinterpret_cast<double*>(w4lds + 8 * PS);   // S_g of each group
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int ng = K / kInt4Group;
-
-    uint32_t em = 0;
-    for (int k = threadIdx.x; k < K; k += kFmtThreads) em = max(em, exp_field(x[k]));
-    em = wave_max_u32(em);
-    if (lane == 0) red[wave] = em;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kFmtWaves; ++i) em = max(em, red[i]);
-    for (int k = threadIdx.x; k < K; k += kFmtThreads) {
-        int d[8];
-        digits55(x[k], em, d);
-        const int at = int4_plane_byte(k);
-#pragma unroll
-        for (int p = 0; p < 8; ++p) planes[p * PS + at] = (uint8_t)(d[p] & 0xff);
-    }
-    for (int g = wave; g < ng; g += kFmtWaves) {
-        int64_t t = fixed55(x[kInt4Group * g + lane], em) + fixed55(x[kInt4Group * g + 64 + lane], em);
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) t += __shfl_xor(t, o, kWave);
-        if (lane == 0) sg[g] = (double)t;
-    }
-    __syncthreads();
-
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, threads = blockDim.x;
+    if (!kCut) S = 1;
+    const int waves = threads / kWave, tiles = waves / S;           // tiles a workgroup works on at once
+    const int ng = K / kInt4Group, np = (ng + 1) / 2;               // groups, pairs of groups
     const int nt = (M + 15) / 16;
     const int items = reps * nt;                  // < 2^31, checked by the host
-    const int total_waves = gridDim.x * kFmtWaves;
+    const int slot = wave / S, seg = wave % S;
+    const int p0 = kCut ? np * seg / S : 0, p1 = kCut ? np * (seg + 1) / S : np;      // the wave's pairs
+
     const int n = lane & 15, kq = lane >> 4;
     const bool low = (lane & 8) == 0;
     const int c = kq + 4 * ((lane >> 3) & 1);     // the lane's 16-byte chunk of a group pair
-    const uint8_t* const arow = planes + (lane & 7) * PS + 16 * kq;
     const int64_t rowbytes = K / 2;
-    const bool vec = vec_scales && (ng % 4) == 0;
-    const double unit = ldexp(1.0, (int)em - 181);
-    for (int it = blockIdx.x * kFmtWaves + wave; it < items; it += total_waves) {
+    uint4 va[U], vb[U];
+    const uint8_t *pA, *pB;
+    const float* srow;
+    auto rows = [&](int it) {                     // rows past M repeat the last one (never stored)
         const int rep = it / nt, tile = it - rep * nt;
         const uint8_t* const wc = w + (int64_t)(rep % n_copies) * copy_stride;
-        // rows past M repeat the last one (never stored)
         const int rA = min(16 * tile + (lane & 7), M - 1), rB = min(16 * tile + 8 + (lane & 7), M - 1);
-        const uint8_t* const pA = wc + (int64_t)rA * rowbytes + 16 * c;
-        const uint8_t* const pB = wc + (int64_t)rB * rowbytes + 16 * c;
-        const float* const srow = scale + (int64_t)min(16 * tile + n, M - 1) * ng;
+        pA = wc + (int64_t)rA * rowbytes + 16 * c;
+        pB = wc + (int64_t)rB * rowbytes + 16 * c;
+        srow = scale + (int64_t)min(16 * tile + n, M - 1) * ng;
+    };
+    auto load = [&](int q0) {                     // pairs q0 .. q0 + U - 1 of the wave's
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (q0 + u < p1 && 2 * (q0 + u) + (c >> 2) < ng) {      // the group this lane's chunk is in
+                va[u] = ldg16_stream(pA + 128 * (int64_t)(q0 + u));
+                vb[u] = ldg16_stream(pB + 128 * (int64_t)(q0 + u));
+            }
+        }
+    };
+    int base = blockIdx.x * tiles;                // first tile of the workgroup's round
+    if (kCut && base + slot < items) {
+        rows(base + slot);
+        load(p0);
+    }
+
+    // the digit planes: each thread's first eight elements stay in registers between the passes
+    uint32_t em = 0;
+    float xv[8];
+    auto load8 = [&](int k) {
+        const float4 f0 = *reinterpret_cast<const float4*>(x + k), f1 = *reinterpret_cast<const float4*>(x + k + 4);
+        xv[0] = f0.x; xv[1] = f0.y; xv[2] = f0.z; xv[3] = f0.w;
+        xv[4] = f1.x; xv[5] = f1.y; xv[6] = f1.z; xv[7] = f1.w;
+    };
+    for (int k = 8 * (int)threadIdx.x; k < K; k += 8 * threads) {
+        load8(k);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) em = max(em, exp_field(xv[i]));
+    }
+    const bool one = K <= 8 * threads;            // xv still holds them
+    em = wave_max_u32(em);
+    if (lane == 0) red[wave] = em;
+    __syncthreads();
+    for (int i = 0; i < waves; ++i) em = max(em, red[i]);
+    for (int k = 8 * (int)threadIdx.x; k < K; k += 8 * threads) {
+        if (!one) load8(k);
+        uint64_t X[8];
+        int64_t t = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            X[i] = (uint64_t)fixed55(xv[i], em);
+            t += (int64_t)X[i];
+        }
+        uint8_t* const at = planes + int4_plane_byte8(k);
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {             // digit p as digits55 has it, a plane at a time (registers)
+            uint32_t d[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                d[i] = (uint32_t)(X[i] >> (49 - 7 * p)) & 127u;
+                if (p == 0) d[i] = (d[i] ^ 64u) - 64u;              // the top digit is signed
+            }
+            *reinterpret_cast<uint2*>(at + p * PS) =
+                make_uint2(pack4(d[0], d[2], d[4], d[6]), pack4(d[1], d[3], d[5], d[7]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // S_g: 16 consecutive threads hold a group
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) t += __shfl_xor(t, o, 16);
+        if ((k & (kInt4Group - 1)) == 0) sg[k / kInt4Group] = (double)t;
+    }
+    __syncthreads();
+
+    const uint8_t* const arow = planes + (lane & 7) * PS + 16 * kq;
+    const double unit = ldexp(1.0, (int)em - 181);
+    int round = 0;
+    for (; base < items; base += gridDim.x * tiles, round ^= 1) {
+        const int it = base + slot;
         double acc = 0.0;
-        for (int g0 = 0; g0 < ng; g0 += U) {
-            uint4 va[U / 2], vb[U / 2];
-            float sc[U];
+        if (it < items) {
+            const bool ahead = kCut && base == (int)blockIdx.x * tiles;       // rows and first pairs requested above
+            if (!ahead) rows(it);
+            for (int q0 = p0; q0 < p1; q0 += U) {
+                if (!ahead || q0 != p0) load(q0);
+                float sc[2 * U];
+                if (vec_scales && (q0 & 1) == 0 && 2 * (q0 + U) <= ng) {    // 16-byte aligned
 #pragma unroll
-            for (int u = 0; u < U / 2; ++u) {
-                if (g0 + 2 * u + (c >> 2) < ng) {        // the group this lane's chunk is in
-                    va[u] = ldg16_stream(pA + 128 * (g0 / 2 + u));
-                    vb[u] = ldg16_stream(pB + 128 * (g0 / 2 + u));
+                    for (int u = 0; u < 2 * U; u += 4) {
+                        float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+                        if (lane < 16) f = *reinterpret_cast<const float4*>(srow + 2 * q0 + u);
+                        sc[u] = f.x; sc[u + 1] = f.y; sc[u + 2] = f.z; sc[u + 3] = f.w;
+                    }
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 2 * U; ++u) sc[u] = (q0 + u / 2 < p1 && 2 * q0 + u < ng) ? srow[2 * q0 + u] : 0.0f;
                 }
-            }
-            if (vec && g0 + U <= ng) {
 #pragma unroll
-                for (int u = 0; u < U; u += 4) {
-                    float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (lane < 16) f = *reinterpret_cast<const float4*>(srow + g0 + u);
-                    sc[u] = f.x; sc[u + 1] = f.y; sc[u + 2] = f.z; sc[u + 3] = f.w;
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < U; ++u) sc[u] = (g0 + u < ng) ? srow[g0 + u] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (g0 + u < ng) {
-                    const int g = g0 + u;
-                    // first group of the pair: low lanes keep their A chunk, high lanes take B from
-                    // lane - 8; second group: low lanes take A from lane + 8, high lanes keep B
-                    const uint4& mine = (u & 1) ? vb[u / 2] : va[u / 2];
-                    const uint4& other = (u & 1) ? va[u / 2] : vb[u / 2];
-                    const bool keep = (u & 1) ? !low : low;
-                    auto pick = [&](uint32_t m, uint32_t o) -> uint32_t {
-                        const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o, 0x128, 0xF, 0xF, false);
-                        return keep ? m : r;                               // 0x128: row_ror:8
-                    };
-                    const uint32_t q0 = pick(mine.x, other.x) ^ 0x88888888u, q1 = pick(mine.y, other.y) ^ 0x88888888u;
-                    const uint32_t q2 = pick(mine.z, other.z) ^ 0x88888888u, q3 = pick(mine.w, other.w) ^ 0x88888888u;
-                    const i32x4_t b0 = {(int)(q0 & 0x0F0F0F0Fu), (int)((q0 >> 4) & 0x0F0F0F0Fu),
-                                        (int)(q1 & 0x0F0F0F0Fu), (int)((q1 >> 4) & 0x0F0F0F0Fu)};
-                    const i32x4_t b1 = {(int)(q2 & 0x0F0F0F0Fu), (int)((q2 >> 4) & 0x0F0F0F0Fu),
-                                        (int)(q3 & 0x0F0F0F0Fu), (int)((q3 >> 4) & 0x0F0F0F0Fu)};
-                    const uint4 a0 = *reinterpret_cast<const uint4*>(arow + kInt4Group * g);
-                    const uint4 a1 = *reinterpret_cast<const uint4*>(arow + kInt4Group * g + 64);
-                    i32x4_t cc = mfma_i8(i32x4_t{(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w}, b0, i32x4_t{0, 0, 0, 0});
-                    cc = mfma_i8(i32x4_t{(int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w}, b1, cc);
-                    // lane n: digits 0-3 of row n, lane n + 16: digits 4-7 (each sum < 2^18, exact)
-                    const double half = ((double)cc[0] * 2097152.0 + (double)cc[1] * 16384.0) +
-                                        ((double)cc[2] * 128.0 + (double)cc[3]);
-                    const double v = fma(half, 268435456.0, partner64<16>(half)) - 8.0 * sg[g];
-                    acc = fma(v, (double)sc[u], acc);
+                for (int u = 0; u < 2 * U; ++u) {
+                    const int g = 2 * q0 + u;
+                    if (q0 + u / 2 < p1 && g < ng) {
+                        // first group of the pair: low lanes keep their A chunk, high lanes take B from
+                        // lane - 8; second group: low lanes take A from lane + 8, high lanes keep B
+                        const uint4& mine = (u & 1) ? vb[u / 2] : va[u / 2];
+                        const uint4& other = (u & 1) ? va[u / 2] : vb[u / 2];
+                        const bool keep = (u & 1) ? !low : low;
+                        auto pick = [&](uint32_t m, uint32_t o) -> uint32_t {
+                            const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o, 0x128, 0xF, 0xF, false);
+                            return keep ? m : r;                               // 0x128: row_ror:8
+                        };
+                        const uint32_t q0w = pick(mine.x, other.x) ^ 0x88888888u, q1w = pick(mine.y, other.y) ^ 0x88888888u;
+                        const uint32_t q2w = pick(mine.z, other.z) ^ 0x88888888u, q3w = pick(mine.w, other.w) ^ 0x88888888u;
+                        const i32x4_t b0 = {(int)(q0w & 0x0F0F0F0Fu), (int)((q0w >> 4) & 0x0F0F0F0Fu),
+                                            (int)(q1w & 0x0F0F0F0Fu), (int)((q1w >> 4) & 0x0F0F0F0Fu)};
+                        const i32x4_t b1 = {(int)(q2w & 0x0F0F0F0Fu), (int)((q2w >> 4) & 0x0F0F0F0Fu),
+                                            (int)(q3w & 0x0F0F0F0Fu), (int)((q3w >> 4) & 0x0F0F0F0Fu)};
+                        const uint4 a0 = *reinterpret_cast<const uint4*>(arow + kInt4Group * g);
+                        const uint4 a1 = *reinterpret_cast<const uint4*>(arow + kInt4Group * g + 64);
+                        i32x4_t cc = mfma_i8(i32x4_t{(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w}, b0, i32x4_t{0, 0, 0, 0});
+                        cc = mfma_i8(i32x4_t{(int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w}, b1, cc);
+                        // lane n: digits 0-3 of row n, lane n + 16: digits 4-7 (each sum < 2^18, exact)
+                        const double half = ((double)cc[0] * 2097152.0 + (double)cc[1] * 16384.0) +
+                                            ((double)cc[2] * 128.0 + (double)cc[3]);
+                        const double v = fma(half, 268435456.0, partner64<16>(half)) - 8.0 * sg[g];
+                        acc = fma(v, (double)sc[u], acc);
+                    }
                 }
             }
         }
-        if (lane < 16 && 16 * tile + n < M) y[(int64_t)(rep % n_copies) * M + 16 * tile + n] = (float)(acc * unit);
+        if constexpr (kCut) {
+            // the waves' partial sums of a tile, added in order by its first wave; two buffers, so
+            // that one barrier a round is enough
+            if (lane < 16) part[round][wave][lane] = acc;
+            __syncthreads();
+            if (seg == 0 && lane < 16)
+                for (int i = 1; i < S; ++i) acc += part[round][wave + i][lane];
+        }
+        if (seg == 0 && it < items && lane < 16) {
+            const int rep = it / nt, row = 16 * (it - rep * nt) + n;
+            if (row < M) y[(int64_t)(rep % n_copies) * M + row] = (float)(acc * unit);
+        }
     }
 }
 
 int launch_int4_t(const float* x, const uint8_t* w, int64_t copy_stride, int n_copies, const float* scale, float* y,
                   int M, int K, int reps, hipStream_t stream) {
     const int64_t items = (int64_t)reps * ((M + 15) / 16);
-    const int64_t want = (items + kFmtWaves - 1) / kFmtWaves;
-    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(want, 8 * device_cu_count()));
-    const size_t lds = (size_t)8 * (K + 16) + sizeof(double) * (K / kInt4Group);   // <= 132 KB (K <= 16384)
-    if (lds > 65536) {
-        static bool raised[64] = {false};          // per device: the limit is the current device's
+    const int np = (K / kInt4Group + 1) / 2;
+    // waves per tile: enough for eight waves a CU, each with a pair of groups at least, then no more
+    // than the waves that this leaves the same most pairs
+    int S = (int)std::min<int64_t>((8 * (int64_t)device_cu_count() + items - 1) / items, std::min(np, kW4MaxWaves));
+    const int per = (np + S - 1) / S;
+    S = (np + per - 1) / per;
+    const int tiles = std::max(1, 4 / S);         // tiles a workgroup works on at once
+    const int threads = S * tiles * kWave;
+    // at most 32 waves a CU (16 in cut tiles), each with the same number of tiles
+    const int64_t most = std::max<int64_t>(1, (S > 1 ? 16 : 32) * (int64_t)device_cu_count() / (S * tiles));
+    const int64_t want = (items + tiles - 1) / tiles;
+    const int64_t rounds = (want + most - 1) / most;
+    const int grid = (int)((want + rounds - 1) / rounds);
+    auto lds_bytes = [](size_t k) { return 8 * (k + 16) + sizeof(double) * (k / kInt4Group); };
+    const size_t lds = lds_bytes((size_t)K);
+    const auto kernel = S > 1 ? int4_gemv_kernel<true> : int4_gemv_kernel<false>;
+    if (lds > 57344) {                             // with the kernel's static 4 KB past the default limit
+        static bool raised[2][64] = {};            // per device: the limit is the current device's
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-        if (!raised[dev]) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(int4_gemv_kernel),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (!raised[S > 1][dev]) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(16384));
             if (e != hipSuccess) return set_error(MQ_ERR_HIP, "int4_gemv: %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-            raised[dev] = true;
+            raised[S > 1][dev] = true;
         }
     }
-    const bool vec_scales = ((uintptr_t)scale % 16) == 0;
-    hipLaunchKernelGGL(int4_gemv_kernel, dim3(grid), dim3(kFmtThreads), lds, stream,
-                       x, w, copy_stride, n_copies, scale, y, M, K, reps, vec_scales);
+    const bool vec_scales = ((uintptr_t)scale % 16) == 0 && (K / kInt4Group) % 4 == 0;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream,
+                       x, w, copy_stride, n_copies, scale, y, M, K, reps, S, vec_scales);
     return check_launch("int4_gemv");
 }
 

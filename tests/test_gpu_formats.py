@@ -103,6 +103,22 @@ def test_int4_gemv_parity(mq, dev, shape):
     assert _rel(y.cpu().double().numpy(), ref) <= 1e-5
 
 
+@pytest.mark.parametrize("shape", [(16, 128), (17, 256), (16, 640), (33, 2944), (1024, 3072), (2048, 6144), (16, 16384),
+                                   (6144, 1024), (40000, 384), (70000, 128)], ids=str)
+def test_int4_gemv_k_cut_and_rounds(mq, dev, shape):
+    """Few row tiles (each cut along K over up to 16 waves, odd group counts included) to many
+    (several rounds per workgroup): fp64 sums of exact products rounded once to fp32, so within
+    2^-24 of the float64 product plus fp64 rounding."""
+    M, K = shape
+    print(f"int4 gemv {M}x{K}", flush=True)
+    q, s = of.quantize_int4_groups(_weights(M, K, seed=M + K))
+    x = torch.randn(K, generator=torch.Generator().manual_seed(K + 2), dtype=torch.float32)
+    y = mq.int4_gemv(x.to(dev), q.to(dev), s.to(dev)).cpu().double().numpy()
+    ref = of.matvec_f64(of.dequant_int4(q, s), x)
+    assert _rel(y, ref) <= 2.0 ** -24
+    assert np.abs(y - ref).max() <= 2.0 ** -24 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("shape", [(64, 1024), (40, 384)], ids=str)
 def test_int4_gemv_one_hot_and_scale_layouts(mq, dev, shape):
     """One-hot activations read single dequantized weights back exactly (s * q is exact in
