@@ -35,6 +35,7 @@
 // the decode step of the last prompt token, as in the reference's loop. A phase's work
 // items (positions or product tiles) are dealt round-robin over the workgroups.
 #include <algorithm>
+#include <type_traits>
 
 #include "attention.h"
 #include "decode_common.h"
@@ -51,8 +52,10 @@ constexpr int kFThreads = 256;
 constexpr int kWtBytes = 128 * 1024;       // most weight bytes a product's row tile holds in LDS
 
 // Chunk workspace for Pp positions (a multiple of kTileP). Digit planes are laid out
-// [K block][position][plane][64 bytes], so that the MFMA A operand of a position pair
-// and K block (16 rows of 64 bytes) is 1 KB of contiguous memory.
+// [K block of 64][position pair][16 bytes of K][position of the pair][plane][16 bytes]: the
+// MFMA A operand of a pair and K block is 1 KB in lane order, so that its load touches each cache
+// line once. (As [position][plane][64 bytes] each quarter of a load touched all eight lines: the down
+// product, the most load-bound, took 23.0 us at 512 positions and 6.5 at 77, now 17.0 and 4.8.)
 struct PfLayout {
     size_t sync, hid, x, q, m, dig, emax, tok, total;
 };
@@ -141,16 +144,42 @@ __device__ __forceinline__ T* pf_buf(const PfArgs& a, size_t off) {
     return reinterpret_cast<T*>(a.ws + off);
 }
 
-// Digit planes of v (4 consecutive elements k0 .. k0 + 3 of position p) into the
-// chunk's plane buffer.
-__device__ __forceinline__ void store_digits4(uint8_t* dig, int Pp, int p, int k0, const float (&v)[4], uint32_t emax) {
+// x[j] of lane i of each quad becomes x[i] of lane j.
+__device__ __forceinline__ void quad_transpose(uint32_t (&x)[4], int lane) {
+    auto swap = [&](uint32_t& lo, uint32_t& hi, bool odd, auto ctrl) {
+        const uint32_t give = odd ? lo : hi;
+        const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, decltype(ctrl)::value, 0xF, 0xF, false);
+        if (odd) lo = got;
+        else hi = got;
+    };
+    const std::integral_constant<int, 0xB1> xor1{};        // quad_perm [1,0,3,2]
+    const std::integral_constant<int, 0x4E> xor2{};        // quad_perm [2,3,0,1]
+    swap(x[0], x[1], lane & 1, xor1);
+    swap(x[2], x[3], lane & 1, xor1);
+    swap(x[0], x[2], lane & 2, xor2);
+    swap(x[1], x[3], lane & 2, xor2);
+}
+
+// Digit planes of v (4 consecutive elements k0 .. k0 + 3 of position p, k0 = 4 t for thread t plus
+// a multiple of 1024) into the chunk's plane buffer. The quad's four threads hold 16 elements, a
+// 16-byte piece of each of the 8 planes, 128 bytes in all: thread j of the quad stores planes 2j
+// and 2j + 1.
+__device__ __forceinline__ void store_digits4(uint8_t* dig, int Pp, int p, int k0, const float (&v)[4], uint32_t emax,
+                                              int lane) {
     int d[4][8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) digits55(v[i], emax, d[i]);
-    uint8_t* base = dig + ((size_t)(k0 / 64) * Pp + p) * 512 + (k0 % 64);
+    uint32_t even[4], odd[4];
 #pragma unroll
-    for (int pl = 0; pl < 8; ++pl)
-        *reinterpret_cast<uint32_t*>(base + 64 * pl) = pack4(d[0][pl], d[1][pl], d[2][pl], d[3][pl]);
+    for (int j = 0; j < 4; ++j) {
+        even[j] = pack4(d[0][2 * j], d[1][2 * j], d[2][2 * j], d[3][2 * j]);
+        odd[j] = pack4(d[0][2 * j + 1], d[1][2 * j + 1], d[2][2 * j + 1], d[3][2 * j + 1]);
+    }
+    quad_transpose(even, lane);
+    quad_transpose(odd, lane);
+    uint8_t* base = dig + ((size_t)(k0 / 64) * Pp + (p & ~1)) * 512 + 256 * ((k0 % 64) / 16) + 128 * (p & 1) + 32 * (lane & 3);
+    reinterpret_cast<uint4*>(base)[0] = make_uint4(even[0], even[1], even[2], even[3]);
+    reinterpret_cast<uint4*>(base)[1] = make_uint4(odd[0], odd[1], odd[2], odd[3]);
 }
 
 // Largest exponent field over a workgroup of kFThreads threads (uniform result).
@@ -230,7 +259,7 @@ __device__ void pf_digits(const PfArgs& a, int p, PfShared& sh) {
     e = block_max_u32(e, rede, wave, lane, kFThreads / kWave);
     uint8_t* dig = pf_buf<uint8_t>(a, L.dig);
 #pragma unroll
-    for (int g = 0; g < G; ++g) store_digits4(dig, a.Pp, p, 1024 * g + 4 * t, n[g], e);
+    for (int g = 0; g < G; ++g) store_digits4(dig, a.Pp, p, 1024 * g + 4 * t, n[g], e, lane);
     if (t == 0) pf_buf<uint32_t>(a, L.emax)[p] = e;
 }
 
@@ -411,7 +440,7 @@ __device__ void pf_gemm(const PfArgs& a, int rt, int pt, PfShared& sh) {
             resx[u] = *reinterpret_cast<const float2*>(pf_buf<float>(a, L.x) + (size_t)pj[u] * kFH + 32 * rt + 2 * l16);
         }
     }
-    const uint8_t* abase = pf_buf<uint8_t>(a, L.dig) + (size_t)p0 * 512 + l16 * 64 + 16 * kq;
+    const uint8_t* abase = pf_buf<uint8_t>(a, L.dig) + (size_t)p0 * 512 + 16 * lane;
     const size_t kstride = (size_t)a.Pp * 512;
 
     i32x4_t A[D][NP];
@@ -549,36 +578,41 @@ __device__ void pf_gemm(const PfArgs& a, int rt, int pt, PfShared& sh) {
     }
 }
 
-// The product's share of workgroup g: one row tile (the one prefetched, rt = g % NRT) against
-// position tiles grp, grp + groups, ... With NRT a multiple of 8 the groups of a row tile lie on
-// one XCD, so its weights come from HBM once. A grid smaller than NRT takes its further row
-// tiles' weights inside the phase. Position tiles hold 32 positions or, when that leaves fewer
+// The product's share of workgroup v: one row tile (the one prefetched, rt = v % NRT) against
+// position tiles grp = v / NRT, grp + groups, ... The workgroups are numbered XCD by XCD, so an
+// XCD holds few groups: the digit planes of its positions (up to 1.5 MB per 64 positions) stay in
+// its L2 while its row tiles pass over them, and what every XCD reads is the weights, during the
+// phases before. (With a row tile's groups on one XCD instead, all planes went through every L2:
+// the prefill took 2.27 instead of 2.19 ms at 77 positions, 4.58 instead of 4.44 at 512.) A grid smaller than NRT takes its further row tiles' weights inside the phase. Position tiles hold 32 positions or, when that leaves fewer
 // rounds' work per workgroup, 16: a 16-position tile takes about 3/5 of a 32-position one's time
 // (QKV 8.3 against 13.7 us, gate|up 6.2 against 9.6 us, one tile per workgroup).
 template <int EPI>
 __device__ __forceinline__ int pf_groups(int G) { return max(G / GemmShape<EPI>::NRT, 1); }
 
+// Workgroup g's place in the order XCD by XCD (workgroups are dealt round-robin over 8 XCDs).
+__device__ __forceinline__ int pf_place(int G, int g) { return (g % kPfXcd) * (G / kPfXcd) + g / kPfXcd; }
+
 template <int EPI>
-__device__ __forceinline__ bool pf_has_tile(const PfArgs& a, int G, int g) {
-    return g / GemmShape<EPI>::NRT < min(pf_groups<EPI>(G), (a.P + 15) / 16);
+__device__ __forceinline__ bool pf_has_tile(const PfArgs& a, int G, int v) {
+    return v / GemmShape<EPI>::NRT < min(pf_groups<EPI>(G), (a.P + 15) / 16);
 }
 
 // Issue the loads of workgroup g's row tile of a layer's product.
 template <int EPI>
 __device__ __forceinline__ void pf_prefetch(const PfArgs& a, int layer, PfShared& sh) {
-    const int G = (int)gridDim.x, g = pf_fresh_uniform((int)blockIdx.x);
-    if (pf_has_tile<EPI>(a, G, g)) pf_load_weights<EPI>(a, layer, g % GemmShape<EPI>::NRT, sh);
+    const int G = (int)gridDim.x, v = pf_place(G, pf_fresh_uniform((int)blockIdx.x));
+    if (pf_has_tile<EPI>(a, G, v)) pf_load_weights<EPI>(a, layer, v % GemmShape<EPI>::NRT, sh);
 }
 
 template <int EPI>
 __device__ __forceinline__ void pf_product(const PfArgs& a, PfShared& sh) {
     constexpr int NRT = GemmShape<EPI>::NRT;
-    const int G = (int)gridDim.x, g = pf_fresh_uniform((int)blockIdx.x);
-    if (!pf_has_tile<EPI>(a, G, g)) return;
-    const int groups = pf_groups<EPI>(G), grp = g / NRT;
+    const int G = (int)gridDim.x, v = pf_place(G, pf_fresh_uniform((int)blockIdx.x));
+    if (!pf_has_tile<EPI>(a, G, v)) return;
+    const int groups = pf_groups<EPI>(G), grp = v / NRT;
     const int n32 = (a.P + 31) / 32, n16 = (a.P + 15) / 16;
     const bool small = 3 * ((n16 + groups - 1) / groups) < 5 * ((n32 + groups - 1) / groups);
-    for (int rt = g % NRT; rt < NRT; rt += G) {
+    for (int rt = v % NRT; rt < NRT; rt += G) {
         if (rt >= G) {                      // not the prefetched tile (uniform)
             __syncthreads();
             pf_load_weights<EPI>(a, a.layer, rt, sh);
