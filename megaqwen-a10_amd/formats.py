@@ -60,22 +60,26 @@ def _shapes(x, w, scale, int4: bool, copies: bool):
         raise TypeError(f"w must be a uint8 {'[n, M, Kw]' if copies else '[M, Kw]'} tensor")
     M, Kw = w.shape[-2:]
     K = 2 * Kw if int4 else Kw
-    if x.dtype != torch.float32 or tuple(x.shape) != (K,):
+    if x.dtype != torch.float32 or x.shape != (K,):
         raise TypeError(f"x must be fp32 [{K}]")
     want = (M, K // INT4_GROUP) if int4 else (M,)
-    if scale.dtype != torch.float32 or tuple(scale.shape) != want:
+    if scale.dtype != torch.float32 or scale.shape != want:
         raise TypeError(f"scale must be fp32 {list(want)}")
-    _check_dev(x=x, w=w, scale=scale)
+    if not (x.is_cuda and w.is_cuda and scale.is_cuda and x.is_contiguous() and w.is_contiguous()
+            and scale.is_contiguous()):
+        _check_dev(x=x, w=w, scale=scale)
     return M, K, Kw
 
 
 def _gemv(fn, x, w, scale, out, int4):
     M, K, _ = _shapes(x, w, scale, int4, False)
+    dev = w.device
     if out is None:
-        out = torch.empty(M, dtype=torch.float32, device=w.device)
-    lib = _lib.load()
-    _lib.check(getattr(lib, fn)(x.data_ptr(), w.data_ptr(), scale.data_ptr(), out.data_ptr(), M, K,
-                                _lib.stream_handle(w.device)), fn)
+        out = torch.empty(M, dtype=torch.float32, device=dev)
+    st = getattr(_lib.load(), fn)(x.data_ptr(), w.data_ptr(), scale.data_ptr(), out.data_ptr(), M, K,
+                                  _lib.stream_handle(dev))
+    if st:
+        _lib.check(st, fn)
     return out
 
 
