@@ -415,10 +415,11 @@ class _DecoderBase:
         return out
 
     PREFILL_CHUNK = 512      # positions per prefill chunk (workspace ~51 KB per position)
-    # shortest prompt prefix generate() sends through prefill(): a prefill of a few positions
-    # takes about 4 ms (one pass over the weights per product phase), as long as 12 decode steps
-    # in one launch, so shorter prompts run as decode steps
-    PREFILL_MIN = 16
+    # shortest prompt prefix generate() sends through prefill(): a prefill of up to 32 positions
+    # takes 1.8 ms whatever their number (nine phases per layer), as decode steps they take 0.33 ms
+    # each. Prefix and first token of 5 positions: 2.01 ms as decode steps, 2.14 with a prefill;
+    # of 6: 2.34 and 2.15; of 7: 2.67 and 2.16
+    PREFILL_MIN = 6
 
     def prefill_supported(self) -> bool:
         """Whether ``prefill`` runs for this decoder (INT8 weights, hidden 1024)."""
