@@ -113,8 +113,10 @@ quantize_int4_groups_kernel(const uint16_t* __restrict__ w, int64_t K, uint8_t* 
 // sums of a tile meet in LDS and are added in wave order. A wave requests its first tile's
 // weights before the workgroup forms the digit planes, eight consecutive elements per
 // thread. Without the cut, and with the planes formed first, byte by byte, from one element per
-// load, single calls took (us, kernel) [1024, 3072] 15.3, [2048, 6144] 29.9, [12288, 2048] 12.4,
-// [6144, 1024] 8.0, [151936, 1024] 28.2; now 6.9, 7.8, 10.2, 6.3 and 21.
+// load, calls took (us, queued back to back, mean of 200) [1024, 3072] 15.9, [2048, 6144] 29.9,
+// [12288, 2048] 12.1, [6144, 1024] 7.1, [151936, 1024] 26.0; now 6.6, 8.5, 9.8, 6.6 and 18.6. Streams of
+// matvecs in one launch (the repeat form) pay for it: 54-55 us before, 55-60 now per step of the
+// Qwen3-0.6B shapes.
 constexpr int kW4Unroll = 4;                      // group pairs whose loads are issued together
 constexpr int kW4MaxWaves = 16;
 
