@@ -820,12 +820,18 @@ __device__ void pf_attention_unit(const PfArgs& a, int x, int pa, int pb, PfShar
 // that the XCD's L2 performs, is that XCD's leader: its agent-scope release writes the XCD's L2
 // back to memory (once per XCD and barrier: one write-back per workgroup, 32 per XCD, cost 26-90
 // us per barrier), then it raises its flag, waits for all eight leaders' flags (eight lanes, one
-// flag each), drops the L2's stale lines, waits for that, and releases its XCD's workgroups through
-// the L2. These drop the stale lines of their own L1 only: every XCD had written its results back
-// before the L2 was cleared, and nothing but weights is read in between. (An agent-scope acquire
-// in every workgroup clears the L2 32 times, the later ones under the phase that has begun: each
-// phase took about 1.3 us longer, a layer 89 instead of 79 us at 77 positions, 173 instead of
-// 165 at 512.) Barrier number b
+// flag each), acquires at agent scope (its L1 and the L2 drop their stale lines), waits for that,
+// and releases its XCD's workgroups through the L2.
+// Every other workgroup empties its own L1, which may hold lines of the exchanged buffers as it read
+// or wrote them in an earlier phase, with an agent-scope acquire too (no narrower one does it: a
+// workgroup-scope acquire is empty where a workgroup runs on one CU). It does so as it arrives, all
+// its loads and stores completed, not once it is released: until then the CU reads nothing but
+// weights and norm gains, which no phase writes (and not even those in the barrier before attention,
+// so that a line they share with a cache row does no harm), so that the L1 holds nothing stale when
+// the leader, after the last XCD's write-back, has cleared the L2 and releases it. The acquire
+// clears the L2 as well, which costs the phase that is ending less than the one that begins: us of a
+// prefill of 2 / 77 / 256 positions with it on arrival 1,986 / 2,292 / 2,775, on release 2,120 /
+// 2,389 / 2,877. Barrier number b
 // completes when an XCD's arrivals reach b times its workgroups and the flags reach b. A wait
 // that expires sets the abort flag, and every later wait of the launch then returns at once,
 // so the grid always drains (the host reports MQ_ERR_TIMEOUT, mq_prefill_check). Needs the
@@ -864,11 +870,13 @@ __device__ __forceinline__ void pf_grid_barrier(PfSync* sy, uint32_t b, uint32_t
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             if (lane == 0) __hip_atomic_store(&mine.lead, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             pf_wait_ge(&sy->xcd[lane % kPfXcd].lead, b, sy, limit);
-            asm volatile("buffer_inv sc1\n\ts_waitcnt vmcnt(0)" ::: "memory");      // this XCD's L2, this CU's L1: done
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            wait_vmem();                    // the lines are gone before the XCD is released
             if (lane == 0) __hip_atomic_store(&mine.released, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         } else {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            wait_vmem();                    // this CU's L1 is empty
             pf_wait_ge(&mine.released, b, sy, limit);
-            asm volatile("buffer_inv sc0\n\ts_waitcnt vmcnt(0)" ::: "memory");      // this CU's L1
         }
     }
     lds_barrier();

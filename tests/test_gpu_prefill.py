@@ -104,6 +104,23 @@ def test_prefill_matches_per_token_steps(full, P):
     _check_rows(_rows(dec, P), want, f"P={P}")
 
 
+@pytest.mark.parametrize("P", [2, 3, 9, 26])
+def test_short_ragged_prefills_through_all_layers(full, P):
+    """Prompts with workgroups that have no position and no product tile: these read little between
+    a layer's queries and K/V rows and the next layer's at the same query addresses, so what the
+    other compute units wrote in between reaches them only through the grid barriers. Two prompts in
+    turn, so that the second's rows differ from what the workspace held."""
+    dec, d, prompt, cfg, _ = full
+    for seed in (200 + P, 300 + P):
+        ids = _tokens(P, cfg.vocab_size, seed)
+        print(f"config-1 model: prefill of {P} positions (seed {seed}) vs {P} decode steps", flush=True)
+        _per_token(dec, ids)
+        want = _rows(dec, P)
+        dec.reset()
+        dec.prefill(ids)
+        _check_rows(_rows(dec, P), want, f"P={P}")
+
+
 @pytest.mark.parametrize("P", [8, 64, 512])
 def test_prefill_matches_oracle(mq, small, P):
     dec, d, prompt, cfg, keep = small

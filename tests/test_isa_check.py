@@ -5,7 +5,10 @@ data-cache stores, atomics, write-back or discard), and no packed fp32
 arithmetic may be formed. The decode kernels copy their per-layer pointer
 tables into LDS before anything else, so none may read LDS before its first
 workgroup barrier (a wave would otherwise read table words another wave has
-not written yet, and dereference what the previous kernel left in LDS).
+not written yet, and dereference what the previous kernel left in LDS). The
+prefill's grid barrier must acquire at agent scope in every workgroup, not in the
+XCDs' leaders alone: the workgroups' L1 caches hold lines of the buffers that the
+phases exchange.
 """
 from __future__ import annotations
 
@@ -58,6 +61,31 @@ def test_decode_kernels_read_lds_only_after_a_barrier(tmp_path):
         seen += sum(1 for n, _ in _kernel_bodies(text) if "decode" in n and "kernel" in n)
         assert not lds_reads_before_first_barrier(text), (src.name, lds_reads_before_first_barrier(text))
     assert seen >= 3
+
+
+def narrow_acquires(text):
+    """Of a kernel with a grid barrier: (cache invalidations narrower than agent scope, agent-scope
+    invalidations, agent-scope write-backs)."""
+    inv = re.findall(r"^\s*buffer_inv\b([^\n;]*)", text, flags=re.M)
+    wb = re.findall(r"^\s*buffer_wbl2\b[^\n;]*sc1", text, flags=re.M)
+    agent = [i for i in inv if "sc1" in i]
+    return len(inv) - len(agent), len(agent), len(wb)
+
+
+def test_prefill_barrier_acquires_at_agent_scope_in_every_workgroup(tmp_path):
+    """Each grid barrier of the prefill has two sides: an XCD's last workgroup (write-back, wait,
+    invalidate, release its XCD) and the others (invalidate, wait). Both invalidations are agent
+    scope's: the workgroup-scope one leaves the L1 as it is outside threadgroup-split mode, which the
+    build does not use."""
+    b = _builder()
+    assert not any("tgsplit" in f for f in b.HIPCC_FLAGS)
+    out = tmp_path / "prefill.s"
+    subprocess.run([b.hipcc(), *b.HIPCC_FLAGS, "--cuda-device-only", "-S", str(b.CSRC / "prefill.hip"), "-o", str(out)],
+                   check=True, capture_output=True)
+    body = [t for n, t in _kernel_bodies(out.read_text()) if "pf_chunk_kernel" in n]
+    assert len(body) == 1
+    narrow, agent, wb = narrow_acquires(body[0])
+    assert wb >= 1 and narrow == 0 and agent == 2 * wb, (narrow, agent, wb)
 
 
 def test_lds_order_check_flags_a_read_before_the_barrier():
