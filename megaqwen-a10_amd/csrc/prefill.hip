@@ -118,7 +118,7 @@ struct PfShared {
     alignas(16) uint16_t qkg[kFD];                     // QKV: the QK-norm gains of the row tile's head
     alignas(16) uint16_t gain[kFH];                    // RMSNorm gains of the next normed digit phase
     double reds[4];
-    uint32_t rede[4];
+    uint32_t rede[2][4];                   // the waves' largest exponents, of a workgroup's positions in turn
 };
 
 enum PfSrc { SRC_EMBED = 0, SRC_HID = 1, SRC_X = 2, SRC_M = 3, SRC_A = 4 };
@@ -198,12 +198,15 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t e, uint32_t* red, int
 // SRC_X: the post-attention residual, post-attention RMSNorm. SRC_M: the SwiGLU
 // output, SRC_A: the attention output (in the query buffer), no norm. The normalized value is fp32(r * rstd * gain) as in the decode
 // step (a10_int8_decode_kernel.cu:54-84, :421-457).
+// `turn` alternates over a workgroup's positions: an un-normed row has one barrier only, behind
+// which a wave may go on to the next position's exponents while another still reads this one's, so
+// these have the other half of rede.
 template <int K, int SRC>
-__device__ void pf_digits(const PfArgs& a, int p, PfShared& sh) {
+__device__ void pf_digits(const PfArgs& a, int p, int turn, PfShared& sh) {
     constexpr int G = K / 1024;            // groups of 4 consecutive elements per thread
     static_assert(SRC == SRC_M || SRC == SRC_A || G == 1, "the normed rows are hidden-sized");
     double* const reds = sh.reds;
-    uint32_t* const rede = sh.rede;
+    uint32_t* const rede = sh.rede[turn];
     const PfLayout L = pf_layout((size_t)a.Pp);
     const int t = pf_fresh(threadIdx.x), lane = t % kWave, wave = t / kWave;
     float v[G][4];
@@ -907,9 +910,9 @@ __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
     for (l = 0; l < a.L; ++l) {
         PfArgs b = a;
         b.layer = l;
-        for (int p = pf_fresh_uniform(g); p < a.P; p += G) {
-            if (l == 0) pf_digits<kFH, SRC_EMBED>(b, p, sh);
-            else pf_digits<kFH, SRC_HID>(b, p, sh);
+        for (int p = pf_fresh_uniform(g), turn = 0; p < a.P; p += G, turn ^= 1) {
+            if (l == 0) pf_digits<kFH, SRC_EMBED>(b, p, turn, sh);
+            else pf_digits<kFH, SRC_HID>(b, p, turn, sh);
         }
         barrier(0, none);
         pf_product<EPI_QKV>(b, sh);
@@ -929,15 +932,15 @@ __global__ void __launch_bounds__(kFThreads, 1) pf_chunk_kernel(PfArgs a) {
             }
         }
         barrier(2, [&] { pf_prefetch<EPI_O>(a, l, sh); });
-        for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFQ, SRC_A>(b, p, sh);
+        for (int p = pf_fresh_uniform(g), turn = 0; p < a.P; p += G, turn ^= 1) pf_digits<kFQ, SRC_A>(b, p, turn, sh);
         barrier(3, [&] { pf_load_gain(a.lw[l].post_attn_layernorm_weight, sh); });
         pf_product<EPI_O>(b, sh);
         barrier(4, [&] { pf_prefetch<EPI_GU>(a, l, sh); });
-        for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFH, SRC_X>(b, p, sh);
+        for (int p = pf_fresh_uniform(g), turn = 0; p < a.P; p += G, turn ^= 1) pf_digits<kFH, SRC_X>(b, p, turn, sh);
         barrier(5, none);
         pf_product<EPI_GU>(b, sh);
         barrier(6, [&] { pf_prefetch<EPI_DOWN>(a, l, sh); });
-        for (int p = pf_fresh_uniform(g); p < a.P; p += G) pf_digits<kFI, SRC_M>(b, p, sh);
+        for (int p = pf_fresh_uniform(g), turn = 0; p < a.P; p += G, turn ^= 1) pf_digits<kFI, SRC_M>(b, p, turn, sh);
         barrier(7, [&] { if (l + 1 < a.L) pf_load_gain(a.lw[l + 1].input_layernorm_weight, sh); });
         pf_product<EPI_DOWN>(b, sh);
         barrier(8, [&] { pf_prefetch<EPI_QKV>(a, l + 1, sh); });

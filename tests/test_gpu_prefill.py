@@ -121,6 +121,20 @@ def test_short_ragged_prefills_through_all_layers(full, P):
         _check_rows(_rows(dec, P), want, f"P={P}")
 
 
+@pytest.mark.parametrize("P", [257, 400])
+def test_two_positions_per_workgroup_through_all_layers(full, P):
+    """More positions than workgroups: a workgroup forms the digits of two positions in turn, each over
+    its own exponent, in every digit phase of every layer (the 2-layer model's last layer has one)."""
+    dec, d, prompt, cfg, _ = full
+    ids = _tokens(P, cfg.vocab_size, 100 + P)
+    print(f"config-1 model: prefill of {P} positions vs {P} decode steps", flush=True)
+    _per_token(dec, ids)
+    want = _rows(dec, P)
+    dec.reset()
+    dec.prefill(ids)
+    _check_rows(_rows(dec, P), want, f"P={P}")
+
+
 @pytest.mark.parametrize("P", [8, 64, 512])
 def test_prefill_matches_oracle(mq, small, P):
     dec, d, prompt, cfg, keep = small
