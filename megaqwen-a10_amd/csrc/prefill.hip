@@ -243,7 +243,8 @@ __device__ void pf_digits(const PfArgs& a, int p, int turn, PfShared& sh) {
         // the gains were loaded into LDS a phase ahead (pf_load_gain), but for the launch's first
         const uint16_t* gain = sh.gain;
         if constexpr (SRC == SRC_EMBED) gain = static_cast<const uint16_t*>(a.lw[a.layer].input_layernorm_weight);
-        const uint2 gu = *reinterpret_cast<const uint2*>(gain + 4 * t);
+        uint2 gu;
+        __builtin_memcpy(&gu, gain + 4 * t, 8);      // the first layer's gains at any element offset
         const float gv[4] = {bf16_bits_to_f32(gu.x & 0xffffu), bf16_bits_to_f32(gu.x >> 16),
                              bf16_bits_to_f32(gu.y & 0xffffu), bf16_bits_to_f32(gu.y >> 16)};
 #pragma unroll
@@ -370,13 +371,21 @@ __device__ __forceinline__ void pf_load_weights(const PfArgs& a, int layer, int 
         }
     }
     const size_t off = (size_t)(lane / 8) * GS::K;
-    for (int i = w - 1; i < RG * KC; i += 3) {
-        const int g = i / KC, kc = i % KC;
-        const int chunk = (lane % 8) ^ (((8 * g + lane / 8) / GS::RPL) % 8);
-        const int8_t* const rows = (EPI == EPI_GU && g >= kGuCh / 8 ? base_up : base) + (size_t)8 * g * GS::K;
-        __builtin_amdgcn_global_load_lds(
-            (const void __attribute__((address_space(1)))*)(rows + off + 128 * kc + 16 * chunk),
-            (void __attribute__((address_space(3)))*)(&sh.wt[(kc * RG + g) * kWave]), 16, 0, 0);
+    auto each = [&](auto&& piece) {         // piece(the lane's 16 bytes, their 1 KB block in LDS)
+        for (int i = w - 1; i < RG * KC; i += 3) {
+            const int g = i / KC, kc = i % KC;
+            const int chunk = (lane % 8) ^ (((8 * g + lane / 8) / GS::RPL) % 8);
+            const int8_t* const rows = (EPI == EPI_GU && g >= kGuCh / 8 ? base_up : base) + (size_t)8 * g * GS::K;
+            piece(rows + off + 128 * kc + 16 * chunk, &sh.wt[(kc * RG + g) * kWave]);
+        }
+    };
+    if (((reinterpret_cast<uintptr_t>(base) | reinterpret_cast<uintptr_t>(base_up)) & 15) == 0) {
+        each([&](const int8_t* src, uint4* dst) {
+            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                             (void __attribute__((address_space(3)))*)dst, 16, 0, 0);
+        });
+    } else {                                // weight matrices at any byte offset
+        each([&](const int8_t* src, uint4* dst) { __builtin_memcpy(dst + lane, src, 16); });
     }
 }
 
@@ -384,8 +393,17 @@ __device__ __forceinline__ void pf_load_weights(const PfArgs& a, int layer, int 
 __device__ __forceinline__ void pf_load_gain(const void* gain, PfShared& sh) {
     const int lane = pf_fresh(threadIdx.x) % kWave;
     if (__builtin_amdgcn_readfirstlane(pf_fresh(threadIdx.x) / kWave) != 1) return;
+    const uint16_t* const src = static_cast<const uint16_t*>(gain) + 2 * lane;
+    if ((reinterpret_cast<uintptr_t>(gain) & 2) == 0) {
 #pragma unroll
-    for (int i = 0; i < kFH; i += 2 * kWave) lds_load4(&sh.gain[i], static_cast<const uint16_t*>(gain) + i + 2 * lane);
+        for (int i = 0; i < kFH; i += 2 * kWave) lds_load4(&sh.gain[i], src + i);
+    } else {                                // a gain vector at an odd element offset
+#pragma unroll
+        for (int i = 0; i < kFH; i += 2 * kWave) {
+            sh.gain[i + 2 * lane] = src[i];
+            sh.gain[i + 2 * lane + 1] = src[i + 1];
+        }
+    }
 }
 
 // The exact values of two position pairs' output tiles. Of pair j's tile lane n (< 16) of each

@@ -232,6 +232,33 @@ def test_long_prompt_three_chunks(small):
     _check_rows(_rows(dec, P), want, f"P={P}")
 
 
+@pytest.mark.parametrize("shift", [1, 2])
+def test_prefill_weights_and_gains_at_any_offset(mq, small, shift):
+    """Weight matrices and norm gains as views 1 or 2 elements into their storage (bytes of int8, 2-byte
+    words of bf16): the same cache rows, bit for bit, as from aligned ones."""
+    dec, d, prompt, cfg, keep = small
+    embed, layers, scales, lm_q, lm_s, fnorm, cos, sin = keep
+
+    def moved(t):
+        flat = torch.empty(t.numel() + shift, dtype=t.dtype, device=t.device)
+        v = flat[shift:].view_as(t)
+        v.copy_(t)
+        return v
+
+    other = mq.A10Int8MegakernelDecoder(embed, [moved(t) for t in layers], scales, lm_q, lm_s, fnorm, cos, sin,
+                                        cfg.num_layers, 512)
+    for P in (7, 300):
+        ids = _tokens(P, cfg.vocab_size, 60 + P)
+        print(f"2-layer model: prefill of {P} positions, weights and gains {shift} elements into their storage", flush=True)
+        dec.reset()
+        dec.prefill(ids)
+        want = _rows(dec, P)
+        other.reset()
+        other.prefill(ids)
+        got = _rows(other, P)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def test_prefill_refuses_before_launch(mq, small):
     dec, d, prompt, cfg, _ = small
     from megaqwen_a10_amd import _lib
