@@ -113,6 +113,45 @@ def test_a10decoder_bf16_generate_is_one_launch(mq, dev):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("name", ["small_int8", "qwen3_0.6b_bf16"])
+def test_one_step_generation(mq, dev, xcd, name):
+    """A launch of a single step (one token in, one out) hands its token out as a longer one does."""
+    dec, d, prompt, cfg, keep = _build(mq, dev, name)
+    dec.set_sampling(0.0)
+    print(f"{name}: one prompt token, one generated token", flush=True)
+    _one_launch_vs_steps(dec, prompt[:1], 1)
+    dec.reset()
+    toks = dec.generate(prompt, 1)
+    assert toks == d["tokens"][:1]
+    for t in d["tokens"][1:4]:                     # one step per call
+        toks = dec.generate(toks, 1)
+        assert toks == [t]
+    del dec, keep
+    torch.cuda.empty_cache()
+
+
+def test_prefilled_prompt_and_one_token_behind_a_deep_cache(mq, dev):
+    """Past the async-wave kernel's range the last prompt token's step, alone in its launch after a
+    prefill, runs on the XCD-aware kernel: the same token and cache rows as one launch per step."""
+    from .test_gpu_decode import _fixture
+    d = _fixture("small_int8")
+    cfg = mq.ModelConfig(**d["config"])
+    state, prompt = mq.random_init_state(cfg, seed=d["seed"], norm_jitter=d["norm_jitter"])
+    S, depth = 6400, 6200
+    cos, sin = mq.precompute_rope_freqs(cfg.head_dim, S, cfg.rope_theta, device=dev)
+    packed = mq.pack_int8(mq.quantize_state(state, cfg, dev), cfg)
+    dec = mq.A10Int8MegakernelDecoder(*packed, cos, sin, cfg.num_layers, S)
+    ids = torch.randint(0, cfg.vocab_size, (20,), generator=torch.Generator().manual_seed(9)).tolist()
+    print(f"2-layer model: {len(ids)} tokens behind {depth} positions, one generated", flush=True)
+    dec.prefill_random_kv(depth, seed=2)
+    want = dec.generate(ids, 1, device_loop=False, batched_prefill=False)
+    dec.prefill_random_kv(depth, seed=2)
+    assert dec.generate(ids, 1) == want
+    assert dec.position() == depth + len(ids)
+    del dec, packed
+    torch.cuda.empty_cache()
+
+
 def test_expired_wait_in_multi_step_launch(mq, dev, xcd):
     dec, d, prompt, cfg, keep = _build(mq, dev, "small_int8")
     dec.set_sampling(0.0)
