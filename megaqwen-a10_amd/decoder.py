@@ -378,7 +378,8 @@ class _DecoderBase:
         """Feed ``prompt_ids`` from the current position and return ``n_tokens`` generated
         tokens, the first being the last prompt step's output (verify_correctness_a10.py:
         323-339). The tokens follow ``set_sampling``. With ``batched_prefill`` (INT8,
-        hidden 1024) and a prompt of more than ``PREFILL_MIN`` tokens, every prompt token but
+        hidden 1024) and a prompt of more than ``PREFILL_MIN`` tokens (a few more behind a
+        filled cache, where a short prefill costs more than its steps), every prompt token but
         the last goes through ``prefill`` (each layer's weights read once for the whole
         prompt); the last prompt token and every generated step are decode steps. With
         ``device_loop`` those steps run in ONE launch and hand their tokens on on the device
@@ -398,7 +399,7 @@ class _DecoderBase:
         if self._pos + len(ids) + n_tokens - 1 > self.max_seq_len:
             raise ValueError(f"position {self._pos} + {len(ids) + n_tokens - 1} steps exceed max_seq_len "
                              f"{self.max_seq_len}")
-        if batched_prefill and len(ids) - 1 >= self.PREFILL_MIN and self.prefill_supported():
+        if batched_prefill and len(ids) - 1 >= self._prefill_min() and self.prefill_supported():
             self.prefill(ids[:-1])
             ids = ids[-1:]
         if device_loop:
@@ -415,11 +416,21 @@ class _DecoderBase:
         return out
 
     PREFILL_CHUNK = 512      # positions per prefill chunk (workspace ~51 KB per position)
-    # shortest prompt prefix generate() sends through prefill(): a prefill of up to 32 positions
-    # takes 1.8 ms whatever their number (nine phases per layer), as decode steps they take 0.33 ms
-    # each. Prefix and first token of 5 positions: 2.01 ms as decode steps, 2.14 with a prefill;
-    # of 6: 2.34 and 2.15; of 7: 2.67 and 2.16
-    PREFILL_MIN = 6
+    # Shortest prompt prefix that goes through prefill() at an empty cache: a prefill of up to 32
+    # positions takes 1.9-2.0 ms whatever their number (nine phases per layer), as decode steps they
+    # take 0.33 ms each. Prompt and first token, us as decode steps / with a prefill: 7 tokens 2,340 /
+    # 2,332, 8 tokens 2,670 / 2,328.
+    PREFILL_MIN = 7
+    # Behind a filled cache one position more for each PREFILL_MIN_STEP cached ones, up to
+    # PREFILL_MIN_DEEP: few positions are few attention items (8 of the 256 workgroups), so a prefill
+    # takes 1.36 us longer per cached position, a decode step 0.03. Behind 1,024 positions: 9 tokens 3,894 /
+    # 3,930; 2,048: 11 tokens 5,274 / 5,277; 4,096: 13 tokens 7,175 / 8,187, 15 tokens 8,272 / 8,191;
+    # 8,192: 17 tokens 17,003 / 13,673 in one launch, 11,139 / 13,653 one by one.
+    PREFILL_MIN_STEP, PREFILL_MIN_DEEP = 576, 16
+
+    def _prefill_min(self) -> int:
+        """Shortest prompt prefix generate() sends through prefill() at the current position."""
+        return min(self.PREFILL_MIN + self._pos // self.PREFILL_MIN_STEP, max(self.PREFILL_MIN, self.PREFILL_MIN_DEEP))
 
     def prefill_supported(self) -> bool:
         """Whether ``prefill`` runs for this decoder (INT8 weights, hidden 1024)."""

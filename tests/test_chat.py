@@ -17,8 +17,11 @@ from types import SimpleNamespace
 
 import pytest
 
+from __graft_entry__ import load_package
+
 from .ckpt import text_of, write_tokenizer
 
+A10Int8MegakernelDecoder = load_package().A10Int8MegakernelDecoder
 V = 64
 
 
@@ -28,7 +31,7 @@ def _rule(fed) -> int:
 
 class FakeSteps:
     """The kernel decoder's surface that A10Chat uses, on the CPU."""
-    PREFILL_MIN = 16
+    PREFILL_MIN = A10Int8MegakernelDecoder.PREFILL_MIN
 
     def __init__(self, max_seq_len=256, prefill=False):
         self.max_seq_len = max_seq_len
@@ -198,9 +201,13 @@ def test_long_prompt_is_prefilled_then_stepped(make_chat):
     assert chat.last_stats["tokens"] == _stepped(prompt, 10)
     # short prompts (fewer than PREFILL_MIN + 1 tokens) run as decode steps
     steps.calls.clear()
-    chat.generate(text_of(prompt[:16]), 10, show_speed=False)
+    n = steps.PREFILL_MIN
+    chat.generate(text_of(prompt[:n]), 10, show_speed=False)
     assert not [c for c in steps.calls if c[0] == "prefill"]
-    assert chat.last_stats["tokens"] == _stepped(prompt[:16], 10)
+    assert chat.last_stats["tokens"] == _stepped(prompt[:n], 10)
+    chat.generate(text_of(prompt[:n + 1]), 10, show_speed=False)
+    assert ("prefill", n) in steps.calls
+    assert chat.last_stats["tokens"] == _stepped(prompt[:n + 1], 10)
 
 
 def test_prompt_truncation(make_chat, capsys):

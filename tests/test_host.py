@@ -282,3 +282,25 @@ def test_wait_host_token(mq):
     assert time.perf_counter() - t0 >= 0.019
     assert "no token" in _lib.last_error() and word.value == -2
     assert lib.mq_wait_host_token(None, -2, 10) == _lib.MQ_ERR_INVALID_ARGUMENT
+
+
+def _route(mq, pos, n, **kw):
+    """Positions that generate() prefills and tokens that it steps for n prompt tokens behind pos."""
+    from megaqwen_a10_amd.decoder import A10Int8MegakernelDecoder
+    dec = object.__new__(A10Int8MegakernelDecoder)
+    dec.dims, dec._pos, dec.max_seq_len = (1024, 3072, 151936), pos, 32768
+    seen = {"prefill": 0, "steps": 0}
+    dec.prefill = lambda ids: seen.update(prefill=len(ids))
+    dec._generate_one_launch = lambda ids, k: seen.update(steps=len(ids)) or [0] * k
+    dec.generate(list(range(n)), 1, **kw)
+    return seen["prefill"], seen["steps"]
+
+
+@pytest.mark.parametrize("pos,least", [(0, 7), (500, 7), (1024, 8), (2048, 10), (4096, 14), (6000, 16), (8192, 16), (30000, 16)])
+def test_short_prompts_behind_a_deep_cache_run_as_steps(mq, pos, least):
+    """A prefill's time grows with the cached positions, most of all for few positions, a step's hardly:
+    the prompt length from which generate() prefills grows with them, up to 16."""
+    assert _route(mq, pos, least) == (0, least)
+    assert _route(mq, pos, least + 1) == (least, 1)
+    assert _route(mq, pos, 40) == (39, 1)
+    assert _route(mq, pos, 40, batched_prefill=False) == (0, 40)
