@@ -95,6 +95,31 @@ def test_one_byte_gemv_row_lengths(mq, dev, M, K):
         assert bool(((y.double() - ref).abs() <= bound + 1e-30).all())
 
 
+def _one_byte_gemv_within_rounding(mq, dev, M, K):
+    """INT8 and FP8 against float64. A lane adds 16 products per 1 KB chunk to one fp32 sum, then six
+    levels add the 64 lanes' and the scale is multiplied on: within (16 chunks + 7) 2^-24 of sum |w x|,
+    which one lane's columns left out or taken from elsewhere exceed many times over."""
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x = torch.randn(K, generator=g, device=dev)
+    s = torch.rand(M, generator=g, device=dev) + 0.5
+    q = torch.randint(-128, 128, (M, K), generator=g, device=dev, dtype=torch.int8)
+    f = (torch.randn((M, K), generator=g, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
+    for y, w in ((mq.int8_gemv(x, q, s), q.double()), (mq.fp8_gemv(x, f.view(torch.uint8), s), f.double())):
+        ref = (w @ x.double()) * s.double()
+        bound = (w.abs() @ x.abs().double()) * s.double() * ((16 * ((K + 1023) // 1024) + 7) * 2.0 ** -24)
+        assert bool(((y.double() - ref).abs() <= bound + 1e-30).all())
+
+
+@pytest.mark.parametrize("M,K", [(70001, 16), (70001, 256), (50000, 1008), (2051, 512), (2049, 8192), (4099, 8208), (1500, 9216),
+                                 (5, 10240), (3001, 10256), (2100, 12288), (2100, 12304), (9, 16384), (2300, 16384),
+                                 (32768, 1024), (32769, 1024)])
+def test_one_byte_gemv_forms(mq, dev, M, K):
+    """Either side of the lines between the kernel's forms, with several items per wave: rows shorter
+    than a chunk, activations in registers and in LDS, matrices that stay in the caches or not."""
+    print(f"gemv {M}x{K}", flush=True)
+    _one_byte_gemv_within_rounding(mq, dev, M, K)
+
+
 def test_int8_gemv_repeatable(mq, dev):
     g = torch.Generator().manual_seed(5)
     q = torch.randint(-127, 128, (4096, 1024), generator=g, dtype=torch.int8).to(dev)
