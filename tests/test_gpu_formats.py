@@ -119,6 +119,27 @@ def test_int4_gemv_k_cut_and_rounds(mq, dev, shape):
     assert np.abs(y - ref).max() <= 2.0 ** -24 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("shape", [(70000, 256), (40, 1152), (9000, 7936), (9000, 8064), (33000, 8064), (5, 10752), (4111, 16256),
+                                   (9000, 16384)], ids=str)
+def test_int4_gemv_long_and_short_rows(mq, dev, shape):
+    """Rows either side of the plane formation's forms (four or eight elements per thread) and of the
+    lengths from which a CU's LDS holds two workgroups' planes, or one's, whose waves then share up to
+    16 tiles, cut or whole; several rounds of tiles. The bound as above."""
+    M, K = shape
+    print(f"int4 gemv {M}x{K}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    q = torch.randint(0, 256, (M, K // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = torch.rand((M, K // 128), generator=g, device=dev) + 0.5
+    x = torch.randn(K, generator=g, device=dev)
+    y = mq.int4_gemv(x, q, s).double()
+    nib = torch.stack((q & 15, q >> 4), -1).view(M, K).to(torch.int8)
+    ref = torch.empty(M, dtype=torch.float64, device=dev)
+    for r in range(0, M, 2048):                      # a group's product and sum in float64, block by block
+        w = ((nib[r:r + 2048] ^ 8) - 8).double().view(-1, K // 128, 128)
+        ref[r:r + 2048] = ((w * x.double().view(1, -1, 128)).sum(-1) * s[r:r + 2048].double()).sum(-1)
+    assert bool(((y - ref).abs() <= 2.0 ** -24 * ref.abs().max()).all())
+
+
 @pytest.mark.parametrize("shape", [(64, 1024), (40, 384)], ids=str)
 def test_int4_gemv_one_hot_and_scale_layouts(mq, dev, shape):
     """One-hot activations read single dequantized weights back exactly (s * q is exact in
