@@ -1,7 +1,7 @@
 """The quantizers' row pass against the element kernels and the oracle (run with -m gpu).
 
 Rows of whole 16-byte loads take the row pass, others (odd lengths, more than 8192 elements,
-views at an odd element offset) the element kernels. The same rows are given to both, the
+views at an odd element offset, few FP8 rows) the element kernels. The same rows are given to both, the
 second time as a view one element into its storage, and must give the same bytes and scales:
 row lengths either side of a wave's 512-element loads and of the register limit, few and many
 rows, and rows of zeros, signed zeros, subnormals, infinities, NaN and the largest values.
@@ -56,9 +56,20 @@ def test_row_pass_matches_element_kernel(mq, dev, fmt, K, M):
     _same((got[0][:n].cpu(), got[1][:n].cpu()), want, f"{fmt} [{M}, {K}] against the oracle")
 
 
-@pytest.mark.parametrize("fmt", ["int8", "fp8", "int4"])
-def test_row_pass_special_values(mq, dev, fmt):
-    K = 1024
+@pytest.mark.parametrize("M", [1023, 1024, 1025])
+@pytest.mark.parametrize("K", [504, 1032, 2040, 4104, 8192])
+def test_fp8_row_pass_and_element_kernel_meet(mq, dev, M, K):
+    """FP8 matrices of fewer rows than four per CU take the element kernel: the same bytes and scales
+    on either side of the line."""
+    print(f"quantize fp8 [{M}, {K}]", flush=True)
+    w = _rows(M, K, dev, K + M)
+    got = _quant(mq, "fp8")(w)
+    _same(got, _quant(mq, "fp8")(_shifted(w)), f"fp8 [{M}, {K}] against the element kernel")
+    many = _quant(mq, "fp8")(torch.cat([w, w, w, w, w]))          # by the row pass on any number of CUs up to 1278
+    _same(got, (many[0][:M], many[1][:M]), f"fp8 [{M}, {K}] against the row pass")
+
+
+def _special_rows(K):
     w = _rows(8, K, torch.device("cpu"), 3).float()
     w[0] = 0.0
     w[1] = -0.0
@@ -68,6 +79,12 @@ def test_row_pass_special_values(mq, dev, fmt):
     w[5] = 3.3e38 * torch.sign(w[5])
     w[6, ::2] = -0.0
     w[7] = float("nan")
-    w = w.to(torch.bfloat16).to(dev)
-    print(f"quantize {fmt}: special values", flush=True)
+    return w.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("copies", [1, 256])
+@pytest.mark.parametrize("fmt", ["int8", "fp8", "int4"])
+def test_row_pass_special_values(mq, dev, fmt, copies):
+    w = _special_rows(1024).to(dev).repeat(copies, 1)
+    print(f"quantize {fmt}: special values, {len(w)} rows", flush=True)
     _same(_quant(mq, fmt)(w), _quant(mq, fmt)(_shifted(w)), fmt)
