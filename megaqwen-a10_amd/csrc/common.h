@@ -427,6 +427,7 @@ __device__ __forceinline__ uint4 ldg16(const void* p) {
     const u32x4_t v = *(const __attribute__((address_space(1))) u32x4_t*)p;
     return make_uint4(v.x, v.y, v.z, v.w);
 }
+constexpr int64_t kLastLevelCache = 256 << 20;       // bytes
 // The same with the non-temporal hint, for the layer weights: every step streams
 // them once (440 MB at the 0.6B shape, more than the 256 MB last-level cache), so
 // they should not displace what is reused from one step to the next there (the

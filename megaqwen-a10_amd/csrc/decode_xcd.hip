@@ -641,16 +641,21 @@ __global__ void __launch_bounds__(kThreads, 1) decode_xcd_kernel(KArgs a) {
         const int64_t rowbytes = (int64_t)H * ES;
         uint4 cur[R], nxt[R];
         float scur = 0.0f, snxt = 0.0f;
-        auto fetch = [&](int b, uint4* dst, float& s) {
+        // A bf16 LM head larger than the last-level cache (0.6B: 311 MB) does not stay there from step to
+        // step, and streamed past it reads faster (496 -> 492 us per step); a smaller one does, beside the
+        // layers' streamed weights, as an 8-bit one (156 MB).
+        const bool past = !kInt8 && a.V * rowbytes > kLastLevelCache;
+        auto request = [&](int b, uint4* dst, auto load) {
 #pragma unroll
             for (int i = 0; i < R; ++i) {
                 const int row = r0 + b * RB + i / CH;
                 dst[i] = make_uint4(0, 0, 0, 0);
-                // a bf16 LM head (311 MB) does not stay in the 256 MB last-level cache from step to
-                // step, and streamed past it reads faster (496 -> 492 us per step at the 0.6B shape); an
-                // 8-bit one (156 MB) does, beside the layers' streamed weights
-                if (row < r1) dst[i] = (kInt8 ? ldg16 : ldg16_stream)(a.lm_w + row * rowbytes + (i % CH) * 1024 + lane * 16);
+                if (row < r1) dst[i] = load(a.lm_w + row * rowbytes + (i % CH) * 1024 + lane * 16);
             }
+        };
+        auto fetch = [&](int b, uint4* dst, float& s) {
+            if (past) request(b, dst, [](const uint8_t* p) { return ldg16_stream(p); });
+            else request(b, dst, [](const uint8_t* p) { return ldg16(p); });
             const int myrow = r0 + b * RB + lane / span;
             s = 1.0f;
             if (kInt8 && myrow < r1) s = gview(a.lm_s)[myrow];
