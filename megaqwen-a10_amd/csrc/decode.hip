@@ -619,6 +619,8 @@ static int launch_t(const KArgs& ka, bool debug, hipStream_t stream, hipEvent_t 
     return MQ_OK;
 }
 
+__global__ void copy_token_kernel(const int* from, int* to) { *to = *from; }
+
 int launch_decode(const mq_decode_args& a, const DecodeShape& s, bool int8, hipStream_t stream, uint32_t* status_out,
                   const GenPlan* plan) {
     if (a.num_layers > kMaxLayers)
@@ -689,7 +691,16 @@ int launch_decode(const mq_decode_args& a, const DecodeShape& s, bool int8, hipS
 
     hipEvent_t t0 = static_cast<hipEvent_t>(a.timing_start), t1 = static_cast<hipEvent_t>(a.timing_stop);
     if (variant == 3) return launch_decode_async(k, debug, s.int4, stream, t0, t1);
-    if (variant == 2) return launch_decode_xcd(k, s, int8, debug, stream, t0, t1);
+    if (variant == 2) {
+        // a plan of one step runs on the per-step form, which stores one token word: the plan's, copied to
+        // the caller's behind it (a second store in that kernel costs every decode step 1.2-1.9 us)
+        const bool one = plan != nullptr && plan->n_steps == 1;
+        if (one) k.out_token = plan->tokens_out;
+        const int st = launch_decode_xcd(k, s, int8, debug, stream, t0, t1);
+        if (st != MQ_OK || !one || a.output_token_id == plan->tokens_out) return st;
+        copy_token_kernel<<<1, 1, 0, stream>>>(plan->tokens_out, a.output_token_id);
+        return check_launch("copy_token_kernel");
+    }
     if (s.H == 1024 && s.I == 3072) {
         return int8 ? launch_t<1024, 3072, Int8W>(k, debug, stream, t0, t1) : launch_t<1024, 3072, Bf16W>(k, debug, stream, t0, t1);
     }

@@ -761,9 +761,6 @@ __global__ void __launch_bounds__(kThreads, 1) decode_xcd_kernel(KArgs a) {
                     if (a.status_out) *a.status_out = flag != 0u ? flag : (wt.dead ? 1u : 0u);
                     __hip_atomic_store(&hdr->xsteps, XS0 + (uint32_t)n_steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     __hip_atomic_store(&hdr->epoch, E0 + (uint32_t)n_steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if constexpr (!kMulti) {       // a plan of one step
-                        if (a.tokens_out != nullptr) *a.tokens_out = chosen;
-                    }
                     if (kDebug && a.trace != nullptr)
                         a.trace[((int64_t)a.L * kTracePoints + 2) * kNWG] = __builtin_amdgcn_s_memrealtime();
                 }

@@ -125,7 +125,7 @@ def test_one_step_generation(mq, dev, xcd, name):
     assert toks == d["tokens"][:1]
     for t in d["tokens"][1:4]:                     # one step per call
         toks = dec.generate(toks, 1)
-        assert toks == [t]
+        assert toks == [t] and int(dec.output_token[0]) == t
     del dec, keep
     torch.cuda.empty_cache()
 
