@@ -22,11 +22,13 @@
 // are eight workgroups a CU, with the registers of the next item's rows given up for it.
 // [100000, 256] 14.7 -> 12.2 us, [100000, 640] 17.8 -> 15.0, [65536, 768] 13.0 -> 11.4.
 //
-// The weights are streamed past the caches where the call's matrices are larger than the L2s
-// (8 x 4 MB), which the next matrix of a model would displace anyway: [151936, 1024] 32.2 -> 28.7 us a
-// call. Smaller ones may still be there from the call before, and streamed they would not stay:
-// called again and again [12288, 2048] 6.9 us streamed and 4.9 not, [6144, 1024] 3.4 and 3.0 (read in
-// turn with others, past every cache, 7.6 and 8.3, 3.7 and 4.2).
+// The weights are streamed past the caches, where the next matrix of a model would displace them
+// anyway ([151936, 1024] 32.2 -> 28.7 us a call), but for matrices of 8 to 32 MB: these may still be in the
+// L2s (8 x 4 MB) from the call before and take much longer from memory. Kernel us, streamed / not:
+// called again and again [12288, 2048] 6.9 / 4.9, [2048, 6144] 6.4 / 5.6, [32768, 1024] 7.4 / 6.3; read in turn
+// with others, past every cache, 7.6 / 8.3, 7.0 / 7.6, 8.5 / 9.3. Up to 8 MB a call is one memory round trip,
+// shorter than its host time: [6144, 1024] again 3.4 / 3.0, in turn 3.7 / 4.2; [4096, 1024] 2.9 / 2.8 and
+// 3.4 / 3.5. Past 32 MB: [49152, 1024] 10.7 / 11.5 and 12.0 / 12.9.
 //
 // Repeat mode (steady-state measurement): one launch computes `reps` matvecs, rep i against
 // weight copy i % n_copies (copies `copy_stride` bytes apart, output row block i % n_copies of
@@ -43,7 +45,7 @@ namespace mq {
 
 constexpr int kGemvThreads = 256;
 constexpr int kGemvWaves = kGemvThreads / kWave;
-constexpr int64_t kGemvCached = 32 << 20;       // bytes of weights that may stay in the L2s
+constexpr int64_t kGemvCachedMin = 8 << 20, kGemvCachedMax = 32 << 20;     // bytes of weights not streamed
 
 // Activations in LDS (rows past 8192 elements)
 constexpr bool gemv_lds(int chmax) { return chmax > 8; }
@@ -142,7 +144,7 @@ int launch_gemv_rows_t(const float* x, const uint8_t* w, int64_t copy_stride, in
     const int64_t even = (waves + kGemvWaves - 1) / kGemvWaves;
     const int grid = (int)(per > 1 ? (even + cus - 1) / cus * cus : even);
     const size_t lds = gemv_lds(CHMAX) ? (size_t)(K + 1023) / 1024 * 4096 : 0;          // at most 64 KB
-    const bool cached = (int64_t)M * K <= kGemvCached / n_copies;
+    const bool cached = (int64_t)M * K > kGemvCachedMin / n_copies && (int64_t)M * K <= kGemvCachedMax / n_copies;
     hipLaunchKernelGGL((cached ? gemv_rows_kernel<F, R, CHMAX, false, kAhead> : gemv_rows_kernel<F, R, CHMAX, true, kAhead>),
                        dim3(grid), dim3(kGemvThreads), lds, stream, x, w, copy_stride, n_copies, scale, y, M, K, reps);
     return check_launch("gemv_rows_kernel");

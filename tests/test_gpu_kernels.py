@@ -103,7 +103,7 @@ def _one_byte_gemv_within_rounding(mq, dev, M, K):
 
 @pytest.mark.parametrize("M,K", [(70001, 16), (70001, 256), (50000, 1008), (2051, 512), (2049, 8192), (4099, 8208), (1500, 9216),
                                  (5, 10240), (3001, 10256), (2100, 12288), (2100, 12304), (9, 16384), (2300, 16384),
-                                 (32768, 1024), (32769, 1024)])
+                                 (8192, 1024), (8193, 1024), (32768, 1024), (32769, 1024)])
 def test_one_byte_gemv_forms(mq, dev, M, K):
     """Either side of the lines between the kernel's forms, with several items per wave: rows shorter
     than a chunk, activations in registers and in LDS, matrices that stay in the caches or not."""
