@@ -9,7 +9,7 @@
 // once, and requests its next row before it works on this one; a grid of at most 8 workgroups
 // per CU strides over the rows (a workgroup per row of 2-byte loads, read twice, spent its
 // time on launching workgroups and issuing loads). [151936, 1024]: INT8 285 -> 84-88 us (5.3-5.6 TB/s,
-// what a copy reaches), FP8 297 -> 101, INT4 (a thread per group) 767 -> 81.
+// what a copy reaches), FP8 297 -> 101-107, INT4 (a thread per group) 767 -> 81-89.
 // The per-element division is three multiply-adds: with r = RN(1 / s), q = RN(w r) and the
 // exact remainder w - q s, RN(q + remainder r) is the correctly rounded w / s (P. Markstein,
 // "Computation of elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
@@ -144,7 +144,7 @@ quantize_rows_wave_kernel(const uint16_t* __restrict__ w, int M, int K, uint8_t*
 
 // Whether the row pass takes these rows: whole lanes of 8 elements, at most 8192 of them, and
 // pointers aligned to a lane's load and store. The other rows go through the formats' element
-// kernels.
+// kernels (and FP8 matrices of few rows, launch_quantize_fp8).
 inline bool quant_rows_fit(const void* w, int K, const void* q, int code_bytes) {
     return K % 8 == 0 && K <= kQRowMaxChunks * kQRowChunk && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
            reinterpret_cast<uintptr_t>(q) % code_bytes == 0;
