@@ -11,10 +11,12 @@
 // time on launching workgroups and issuing loads). [151936, 1024]: INT8 285 -> 84-88 us (5.3-5.6 TB/s,
 // what a copy reaches), FP8 297 -> 101-107, INT4 (a thread per group) 767 -> 81-89.
 // The per-element division is three multiply-adds: with r = RN(1 / s), q = RN(w r) and the
-// exact remainder w - q s, RN(q + remainder r) is the correctly rounded w / s (P. Markstein,
+// remainder w - q s, RN(q + remainder r) is the correctly rounded w / s (P. Markstein,
 // "Computation of elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
-// Dev. 34, 1990). It needs s finite (else the IEEE division is used); where w is so small that
-// the remainder underflows, w / s is below 2^-60 either way and its code is 0.
+// Dev. 34, 1990; his q is within one unit of w / s and the remainder exact, here q can be half a
+// unit further off, and every pair of mantissas that w and s can have was checked). It needs s
+// finite (else the IEEE division is used); where w is so small that the remainder underflows, w / s
+// is below 2^-60 either way and its code is 0.
 #pragma once
 
 #include "common.h"
